@@ -110,6 +110,50 @@ __device__ __forceinline__ void spmv_epilogue(int64_t idx, int64_t row, T acc, T
   }
 }
 
+// The same for one column and V = T in two halves, so that the row's vector
+// entries can be loaded ahead of the row sum (same values, same order).
+template <typename T>
+struct SpmvRow {
+  T sd, x, b, dinv, d, y;
+
+  template <int MODE>
+  __device__ __forceinline__ void load(int64_t row, const T* __restrict__ sdp, const T* __restrict__ xp,
+                                       const T* __restrict__ yp, const T* __restrict__ bp,
+                                       const T* __restrict__ dinvp, const T* __restrict__ dp, T c1) {
+    constexpr bool nt = MODE == kCheb && sizeof(T) == 8;
+    if (sdp) sd = sdp[row];
+    if (sdp || MODE == kJacobi || MODE == kCheb) x = xp[row];
+    if (MODE == kResid || MODE == kJacobi || MODE == kCheb) b = nt ? ntload(bp + row) : bp[row];
+    if (MODE == kAssignScale || MODE == kJacobi || MODE == kCheb) dinv = nt ? ntload(dinvp + row) : dinvp[row];
+    if (MODE == kCheb) d = c1 != T(0) ? (nt ? ntload(dp + row) : dp[row]) : T(0);
+    if (MODE == kAdd) y = yp[row];
+  }
+
+  template <int MODE>
+  __device__ __forceinline__ void store(int64_t row, T acc, T* __restrict__ yp, T* __restrict__ dp,
+                                        T* __restrict__ xn, T c1, T c2) {
+    if (MODE == kAssign) {
+      yp[row] = acc;
+    } else if (MODE == kAssignScale) {
+      yp[row] = acc;
+      const T v = c1 * dinv * acc;
+      xn[row] = v;
+      if (dp) dp[row] = v;
+    } else if (MODE == kResid) {
+      yp[row] = b - acc;
+    } else if (MODE == kAdd) {
+      yp[row] = y + acc;
+    } else if (MODE == kJacobi) {
+      xn[row] = x + c1 * dinv * (b - acc);
+    } else {
+      const T r = dinv * (b - acc);
+      const T dn = (c1 != T(0) ? c1 * d : T(0)) + c2 * r;
+      dp[row] = dn;
+      xn[row] = x + dn;
+    }
+  }
+};
+
 // Single right-hand side: G lanes per row, strided over the row's entries,
 // reduced by a butterfly (fixed order).
 template <typename V, typename T, int G, int MODE>
@@ -276,63 +320,182 @@ struct LdsView {
 
 inline LdsView lds_view(const Csr& A) { return LdsView{A.lds_bs, A.lc.get(), A.lcs.get(), A.lcols.get()}; }
 
-// x at the block's distinct columns into xs (then a block barrier)
-template <typename T>
-__device__ __forceinline__ void lds_stage(const LdsView& L, unsigned blk, const T* __restrict__ x, T* xs) {
-  const int c0 = L.lcs[blk], nc = L.lcs[blk + 1] - c0;
-  for (int t = threadIdx.x; t < nc; t += blockDim.x) xs[t] = x[L.lcols[c0 + t]];
-  __syncthreads();
+// x at the block's distinct columns into xs (then a block barrier), in two
+// halves: the first kStageCols columns of each thread are loaded by begin(),
+// so that loads which do not depend on them can be issued before finish()
+// gathers x.
+constexpr int kStageCols = 4;
+struct LdsStage {
+  int c0, nc;
+  int col[kStageCols];
+
+  __device__ __forceinline__ void begin(const LdsView& L, unsigned blk) {
+    c0 = L.lcs[blk];
+    nc = L.lcs[blk + 1] - c0;
+#pragma unroll
+    for (int j = 0; j < kStageCols; ++j) {
+      const int t = (int)threadIdx.x + j * (int)blockDim.x;
+      if (t < nc) col[j] = L.lcols[c0 + t];
+    }
+  }
+
+  template <typename T>
+  __device__ __forceinline__ void finish(const LdsView& L, const T* __restrict__ x, T* xs) {
+    T v[kStageCols];
+#pragma unroll
+    for (int j = 0; j < kStageCols; ++j)
+      if ((int)threadIdx.x + j * (int)blockDim.x < nc) v[j] = x[col[j]];
+#pragma unroll
+    for (int j = 0; j < kStageCols; ++j) {
+      const int t = (int)threadIdx.x + j * (int)blockDim.x;
+      if (t < nc) xs[t] = v[j];
+    }
+    for (int t = (int)threadIdx.x + kStageCols * (int)blockDim.x; t < nc; t += blockDim.x)
+      xs[t] = x[L.lcols[c0 + t]];
+    __syncthreads();
+  }
+};
+
+// The first HEAD steps of a lane's row (LDS indices and stored values),
+// loaded before the staging barrier: they do not depend on x, so their memory
+// latency runs beside the staging's (list offsets -> columns -> x) instead of
+// after it.  In groups of four, and the remainder of a row that ends there;
+// which loads are issued is the same for the whole wavefront.
+template <typename V, int HEAD>
+struct SliceHead {
+  unsigned c[HEAD > 0 ? HEAD : 1], rc[3];
+  V v[HEAD > 0 ? HEAD : 1], rv[3];
+  int off, w;  // the slice's first element and steps
+};
+
+template <typename V, int HEAD>
+__device__ __forceinline__ void lds_head(SliceHead<V, HEAD>& H, const SellView& S, const LdsView& L, int slice,
+                                         int lane, const V* __restrict__ sv) {
+  H.off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
+  H.w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - H.off) >> 6);
+  const V* vp = sv + H.off + lane;
+  const uint16_t* cp = L.lc + H.off + lane;
+#pragma unroll
+  for (int g = 0; g < HEAD; g += 4) {
+    if (g + 4 <= H.w) {
+#pragma unroll
+      for (int j = g; j < g + 4; ++j) {
+        H.c[j] = ntload(cp + 64 * j);
+        H.v[j] = ntload(vp + 64 * j);
+      }
+    }
+  }
+  if (H.w < HEAD) {
+    const int base = H.w & ~3;
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      if (base + j < H.w) {
+        H.rc[j] = ntload(cp + 64 * (base + j));
+        H.rv[j] = ntload(vp + 64 * (base + j));
+      }
+    }
+  }
 }
 
-// row sum of slice `slice` with x from LDS (same entry order as sell_row_sum)
-template <typename T, typename V = T>
-__device__ __forceinline__ T lds_row_sum(const SellView& S, const LdsView& L, int slice, int lane,
+// value of a stored matrix entry in the working precision: FP64 / FP32 as
+// stored, FP16 kept as its 16-bit pattern (uint16_t)
+template <typename T, typename V>
+__device__ __forceinline__ T sell_cvt(V v) { return (T)v; }
+template <>
+__device__ __forceinline__ float sell_cvt<float, uint16_t>(uint16_t v) {
+  return (float)__builtin_bit_cast(_Float16, v);
+}
+
+// row sum with x from LDS, the head's entries first (same entry order as
+// sell_row_sum)
+template <typename T, typename V, int HEAD>
+__device__ __forceinline__ T lds_row_sum(const SliceHead<V, HEAD>& H, const LdsView& L, int lane,
                                          const V* __restrict__ sv, const T* xs) {
-  const int off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
-  const int w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - off) >> 6);
-  const V* vp = sv + off + lane;
-  const uint16_t* cp = L.lc + off + lane;
   T acc = T(0);
-  int k = 0;
-  for (; k + 4 <= w; k += 4) {
-    const unsigned i0 = ntload(cp + 64 * k), i1 = ntload(cp + 64 * (k + 1)), i2 = ntload(cp + 64 * (k + 2)),
-                   i3 = ntload(cp + 64 * (k + 3));
-    const T v0 = sell_val<T>(vp + 64 * k), v1 = sell_val<T>(vp + 64 * (k + 1)), v2 = sell_val<T>(vp + 64 * (k + 2)),
-            v3 = sell_val<T>(vp + 64 * (k + 3));
-    acc += v0 * xs[i0];
-    acc += v1 * xs[i1];
-    acc += v2 * xs[i2];
-    acc += v3 * xs[i3];
+#pragma unroll
+  for (int g = 0; g < HEAD; g += 4) {
+    if (g + 4 <= H.w) {
+#pragma unroll
+      for (int j = g; j < g + 4; ++j) acc += sell_cvt<T>(H.v[j]) * xs[H.c[j]];
+    }
   }
-  for (; k < w; ++k) acc += sell_val<T>(vp + 64 * k) * xs[ntload(cp + 64 * k)];
+  if (H.w < HEAD) {
+    const int base = H.w & ~3;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      if (base + j < H.w) acc += sell_cvt<T>(H.rv[j]) * xs[H.rc[j]];
+    return acc;
+  }
+  const V* vp = sv + H.off + lane;
+  const uint16_t* cp = L.lc + H.off + lane;
+  int k = HEAD;
+  for (; k + 4 <= H.w; k += 4) {
+    unsigned c[4];
+    V v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      c[j] = ntload(cp + 64 * (k + j));
+      v[j] = ntload(vp + 64 * (k + j));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc += sell_cvt<T>(v[j]) * xs[c[j]];
+  }
+  for (; k < H.w; ++k) acc += sell_cvt<T>(ntload(vp + 64 * k)) * xs[ntload(cp + 64 * k)];
   return acc;
 }
 
+// A block on the LDS-staged copy: L.bs slices, a wavefront each (blocks of
+// more wavefronts use the others for staging only).
+constexpr int kLdsMaxSlices = 8;
+constexpr int kLdsMaxNT = 64 * kLdsMaxSlices;
+
+struct LdsWave {
+  int lane, slice;
+  bool live;    // this wavefront has a slice
+  bool on;      // and this lane one of its rows
+  int64_t pos;  // the lane's row position
+};
+
+__device__ __forceinline__ LdsWave lds_wave(const LdsView& L, unsigned blk, int64_t n, int64_t nslices) {
+  LdsWave w;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  w.lane = threadIdx.x & 63;
+  w.slice = (int)blk * L.bs + wv;
+  w.live = wv < L.bs && w.slice < nslices;
+  w.pos = (int64_t)w.slice * 64 + w.lane;
+  w.on = w.live && w.pos < n;
+  return w;
+}
+
 // SpMV with the fused epilogues on the LDS-staged copy; grid = one block per
-// L.bs slices, dynamic LDS = the largest distinct-column count x sizeof(T)
-template <typename T, int MODE>
-__global__ void __launch_bounds__(kNT) sell_lds_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
-                                                     const T* __restrict__ sv, const T* __restrict__ x,
-                                                     T* __restrict__ y, const T* __restrict__ b,
-                                                     const T* __restrict__ dinv, T* __restrict__ d,
-                                                     T* __restrict__ xn, T c1, T c2) {
+// L.bs slices, dynamic LDS = the largest distinct-column count x sizeof(T).
+// The row's vector entries are loaded before the staging barrier too.
+template <typename T, int MODE, int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) sell_lds_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
+                                                           const T* __restrict__ sv, const T* __restrict__ x,
+                                                           T* __restrict__ y, const T* __restrict__ b,
+                                                           const T* __restrict__ dinv, T* __restrict__ d,
+                                                           T* __restrict__ xn, T c1, T c2) {
   extern __shared__ unsigned char lds_raw[];
   T* xs = reinterpret_cast<T*>(lds_raw);
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  lds_stage<T>(L, blk, x, xs);
-  const int lane = threadIdx.x & 63;
+  const LdsWave w = lds_wave(L, blk, n, nslices);
   const T* sd = sell_diag<T>(S);
-  for (int q = threadIdx.x >> 6; q < L.bs; q += kNT / 64) {
-    const int slice = __builtin_amdgcn_readfirstlane((int)(blk * L.bs + q));
-    if (slice >= nslices) break;
-    T acc = lds_row_sum<T>(S, L, slice, lane, sv, xs);
-    const int64_t pos = (int64_t)slice * 64 + lane;
-    if (pos < n) {
-      const int64_t row = S.srow ? (int64_t)S.srow[pos] : pos;
-      if (sd) acc += sd[row] * x[row];  // the diagonal term, last
-      spmv_epilogue<MODE, T, T>(row, row, acc, y, x, b, dinv, d, xn, c1, c2);
-    }
+  LdsStage G;
+  SliceHead<T, HEAD> H;
+  SpmvRow<T> R;
+  int64_t row = w.pos;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sv);
+  if (w.on) {
+    if (S.srow) row = S.srow[w.pos];
+    R.template load<MODE>(row, sd, x, y, b, dinv, d, c1);
   }
+  G.finish<T>(L, x, xs);
+  if (!w.on) return;
+  T acc = lds_row_sum<T>(H, L, w.lane, sv, xs);
+  if (sd) acc += R.sd * R.x;  // the diagonal term, last
+  R.template store<MODE>(row, acc, y, d, xn, c1, c2);
 }
 
 // G lanes per row (slices of 64 / G rows): each lane sums its strided share
@@ -570,15 +733,16 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Sum of v over the block (fixed order); result valid in thread 0.
-__device__ __forceinline__ double block_sum(double v, double* s_buf) {
+// Sum of v over the block of 64 * waves threads (fixed order); result valid in
+// thread 0.
+__device__ __forceinline__ double block_sum(double v, double* s_buf, int waves = kNT / 64) {
   v = wave_sum(v);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) s_buf[w] = v;
   __syncthreads();
   double r = 0.0;
   if (threadIdx.x == 0)
-    for (int i = 0; i < kNT / 64; ++i) r += s_buf[i];
+    for (int i = 0; i < waves; ++i) r += s_buf[i];
   __syncthreads();
   return r;
 }

@@ -166,6 +166,40 @@ void launch_sell_multi(const Csr& A, int k, const T* x, T* y, const T* b, const 
                                                                            svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2);
 }
 
+constexpr int kLdsHead = 16;         // steps
+constexpr int64_t kLdsHeadRow = 20;  // average row length above which no head is loaded
+
+// Launch on an LDS-staged copy with values of `vsize` bytes: f(head steps,
+// blocks, threads).  Loading the first 16 steps before the staging barrier
+// pays where that latency is exposed, at the price of registers (FP32 48,
+// FP64 66 per lane).  Measured (Chebyshev step, before -> with the head):
+//  * 97^3, blocks of 2 slices: FP32 25.2 -> 20.9 us, FP64 operator + p.q
+//    35.8 -> 31.9 us; 49^3 FP64 7.6 -> 6.6 us;
+//  * 161^3 FP32, blocks of 8: 88.5 -> 76.6 us (505 MB: 6.6 TB/s); FP16 alike;
+//  * FP64 in blocks of 8 fills the memory system anyway and loses a
+//    wavefront per SIMD to the registers: 8, 12, 16 head steps give 88.7,
+//    93.8, 85.0 us at 131 x 150 x 119 against 81.6 us without;
+//  * rows longer than the head (161^3 level 1, ~46 entries): 16.9 us without,
+//    18.5 with; their blocks of 2 slices stage with four wavefronts;
+//  * 2D operators (~7 entries per row) need 8 steps: 1003 x 701 FP64 operator
+//    + p.q 18.2 -> 13.3 us (15.7 with 16 steps' registers);
+//  * fewer blocks than CUs (65^2: 34): a launch is all latency, and the longer
+//    code of the head costs more than it hides (3.25 us against 3.6).
+template <typename Fn>
+void lds_launch(const Csr& A, size_t vsize, Fn&& f) {
+  const unsigned nb = (unsigned)((A.nslices + A.lds_bs - 1) / A.lds_bs);
+  const unsigned nt = 64u * (unsigned)A.lds_bs;
+  const bool lengths = A.srow.size() > 0;  // rows in length order (prolongators)
+  if (nb < 256u || A.nnz > kLdsHeadRow * A.n)
+    f(std::integral_constant<int, 0>{}, nb, nt < 256u ? 256u : nt);
+  else if (A.lds_bs > 2 && vsize == 8)
+    f(std::integral_constant<int, 0>{}, nb, nt);
+  else if (A.nnz <= 8 * A.n && !lengths)
+    f(std::integral_constant<int, 8>{}, nb, nt);
+  else
+    f(std::integral_constant<int, kLdsHead>{}, nb, nt);
+}
+
 // y/xn = f(A x) for k right-hand sides; MODE selects the epilogue.  One RHS
 // uses the sliced-ELL copy when it exists, otherwise CSR with G lanes per row.
 template <typename T, int MODE>
@@ -174,9 +208,10 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
   if (A.n == 0) return;
   const T* val = vals_of<T>(A);
   if (k == 1 && A.nslices > 0 && svals_of<T>(A) && A.lds_bs > 0) {
-    const unsigned nb = (unsigned)((A.nslices + A.lds_bs - 1) / A.lds_bs);
-    sell_lds_kernel<T, MODE><<<nb, kNT, sizeof(T) * (size_t)A.lds_maxc, s>>>(
-        A.n, A.nslices, sell_view(A), lds_view(A), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2);
+    lds_launch(A, sizeof(T), [&](auto head, unsigned nb, unsigned nt) {
+      sell_lds_kernel<T, MODE, head.value><<<nb, nt, sizeof(T) * (size_t)A.lds_maxc, s>>>(
+          A.n, A.nslices, sell_view(A), lds_view(A), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2);
+    });
   } else if (k == 1 && A.nslices > 0 && svals_of<T>(A)) {
     switch (A.sell_g) {
       case 1: launch_sell<T, MODE, 1>(A, x, y, b, dinv, d, xn, c1, c2, s); break;
@@ -292,42 +327,51 @@ __global__ void __launch_bounds__(kNT) sell_smooth_out_kernel(int64_t n, int64_t
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
-// The same on the LDS-staged copy: a block per L.bs slices, r.z partials per block.
-template <int MODE>
-__global__ void __launch_bounds__(kNT) sell_lds_out_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
-                                                         const float* __restrict__ sv, const float* __restrict__ x,
-                                                         const float* __restrict__ b, const float* __restrict__ dinv,
-                                                         const float* __restrict__ d, float c1, float c2,
-                                                         const double* __restrict__ r, double* __restrict__ z,
-                                                         double* __restrict__ partials) {
+// The same on the LDS-staged copy: a block per L.bs slices (a wavefront each),
+// r.z partials per block.
+template <int MODE, int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) sell_lds_out_kernel(
+    int64_t n, int64_t nslices, SellView S, LdsView L, const float* __restrict__ sv, const float* __restrict__ x,
+    const float* __restrict__ b, const float* __restrict__ dinv, const float* __restrict__ d, float c1, float c2,
+    const double* __restrict__ r, double* __restrict__ z, double* __restrict__ partials) {
   extern __shared__ unsigned char lds_raw[];
   float* xs = reinterpret_cast<float*>(lds_raw);
-  __shared__ double s_buf[kNT];
+  __shared__ double s_buf[kLdsMaxNT / 64];
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  lds_stage<float>(L, blk, x, xs);
-  const int lane = threadIdx.x & 63;
-  double part = 0.0;
-  for (int q = threadIdx.x >> 6; q < L.bs; q += kNT / 64) {
-    const int slice = __builtin_amdgcn_readfirstlane((int)(blk * L.bs + q));
-    if (slice >= nslices) break;
-    float acc = lds_row_sum<float>(S, L, slice, lane, sv, xs);
-    const int64_t row = (int64_t)slice * 64 + lane;
-    if (row < n) {
-      if (S.sd32) acc += S.sd32[row] * x[row];  // the diagonal term, last
-      float xn;
-      if (MODE == kJacobi) {
-        xn = x[row] + c1 * dinv[row] * (b[row] - acc);
-      } else {
-        const float rr = ntload(dinv + row) * (ntload(b + row) - acc);
-        const float dn = (c1 != 0.0f ? c1 * ntload(d + row) : 0.0f) + c2 * rr;
-        xn = x[row] + dn;
-      }
-      const double zv = (double)xn;
-      z[row] = zv;
-      part += r[row] * zv;
-    }
+  const LdsWave w = lds_wave(L, blk, n, nslices);
+  const int64_t row = w.pos;
+  SliceHead<float, HEAD> H;
+  float xv = 0.0f, bv = 0.0f, iv = 0.0f, dv = 0.0f, sdv = 0.0f;
+  double rv = 0.0;
+  LdsStage G;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sv);
+  if (w.on) {
+    xv = x[row];
+    bv = ntload(b + row);
+    iv = ntload(dinv + row);
+    if (MODE == kCheb && c1 != 0.0f) dv = ntload(d + row);
+    if (S.sd32) sdv = S.sd32[row];
+    rv = r[row];
   }
-  const double tot = block_sum(part, s_buf);
+  G.finish<float>(L, x, xs);
+  double part = 0.0;
+  float acc = w.on ? lds_row_sum<float>(H, L, w.lane, sv, xs) : float(0);
+  if (w.on) {
+    if (S.sd32) acc += sdv * xv;  // the diagonal term, last
+    float xn;
+    if (MODE == kJacobi) {
+      xn = xv + c1 * iv * (bv - acc);
+    } else {
+      const float rr = iv * (bv - acc);
+      const float dn = (c1 != 0.0f ? c1 * dv : 0.0f) + c2 * rr;
+      xn = xv + dn;
+    }
+    const double zv = (double)xn;
+    z[row] = zv;
+    part = rv * zv;
+  }
+  const double tot = block_sum(part, s_buf, blockDim.x >> 6);
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
@@ -410,78 +454,89 @@ __global__ void __launch_bounds__(kNT) sell_half_out_kernel(int64_t n, int64_t n
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
-// The same two kernels on the LDS-staged copy: a block stages y at its
-// slices' distinct columns once, and every entry reads y from LDS through its
-// 16-bit index (same entries in the same order, so the same sums).
-template <int MODE>
-__global__ void __launch_bounds__(kNT) sell_half_lds_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
-                                                          const uint16_t* __restrict__ sh,
-                                                          const float* __restrict__ diag, const float* __restrict__ y,
-                                                          const float* __restrict__ bh, float* __restrict__ out,
-                                                          float* __restrict__ d, float* __restrict__ yn, float c1,
-                                                          float c2) {
+// The same two kernels on the LDS-staged copy: a block of a wavefront per
+// slice stages y at its slices' distinct columns once, and every entry reads
+// y from LDS through its 16-bit index (same entries in the same order, so the
+// same sums).
+template <int MODE, int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) sell_half_lds_kernel(
+    int64_t n, int64_t nslices, SellView S, LdsView L, const uint16_t* __restrict__ sh, const float* __restrict__ diag,
+    const float* __restrict__ y, const float* __restrict__ bh, float* __restrict__ out, float* __restrict__ d,
+    float* __restrict__ yn, float c1, float c2) {
   extern __shared__ unsigned char lds_raw[];
   float* ys = reinterpret_cast<float*>(lds_raw);
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  lds_stage<float>(L, blk, y, ys);
-  const int lane = threadIdx.x & 63;
-  for (int q = threadIdx.x >> 6; q < L.bs; q += kNT / 64) {
-    const int slice = __builtin_amdgcn_readfirstlane((int)(blk * L.bs + q));
-    if (slice >= nslices) break;
-    const float acc = lds_row_sum<float, uint16_t>(S, L, slice, lane, sh, ys);
-    const int64_t row = (int64_t)slice * 64 + lane;
-    if (row >= n) continue;
-    const float yi = y[row];
-    const float r = ntload(bh + row) - (ntload(diag + row) * yi + acc);
-    if (MODE == kResid) {
-      out[row] = r;
-    } else if (MODE == kJacobi) {
-      yn[row] = yi + c1 * r;
-    } else {
-      const float dn = (c1 != 0.0f ? c1 * ntload(d + row) : 0.0f) + c2 * r;
-      d[row] = dn;
-      yn[row] = yi + dn;
-    }
+  const LdsWave w = lds_wave(L, blk, n, nslices);
+  const int64_t row = w.pos;
+  SliceHead<uint16_t, HEAD> H;
+  float yi = 0.0f, bv = 0.0f, gv = 0.0f, dv = 0.0f;
+  LdsStage G;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sh);
+  if (w.on) {
+    yi = y[row];
+    bv = ntload(bh + row);
+    gv = ntload(diag + row);
+    if (MODE == kCheb && c1 != 0.0f) dv = ntload(d + row);
+  }
+  G.finish<float>(L, y, ys);
+  float acc = w.on ? lds_row_sum<float>(H, L, w.lane, sh, ys) : float(0);
+  if (!w.on) return;
+  const float r = bv - (gv * yi + acc);
+  if (MODE == kResid) {
+    out[row] = r;
+  } else if (MODE == kJacobi) {
+    yn[row] = yi + c1 * r;
+  } else {
+    const float dn = (c1 != 0.0f ? c1 * dv : 0.0f) + c2 * r;
+    d[row] = dn;
+    yn[row] = yi + dn;
   }
 }
 
-template <int MODE>
-__global__ void __launch_bounds__(kNT) sell_half_lds_out_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
-                                                              const uint16_t* __restrict__ sh,
-                                                              const float* __restrict__ diag,
-                                                              const float* __restrict__ sd,
-                                                              const float* __restrict__ y,
-                                                              const float* __restrict__ bh,
-                                                              const float* __restrict__ d, float c1, float c2,
-                                                              const double* __restrict__ r64, double* __restrict__ z,
-                                                              double* __restrict__ partials) {
+template <int MODE, int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) sell_half_lds_out_kernel(
+    int64_t n, int64_t nslices, SellView S, LdsView L, const uint16_t* __restrict__ sh, const float* __restrict__ diag,
+    const float* __restrict__ sd, const float* __restrict__ y, const float* __restrict__ bh,
+    const float* __restrict__ d, float c1, float c2, const double* __restrict__ r64, double* __restrict__ z,
+    double* __restrict__ partials) {
   extern __shared__ unsigned char lds_raw[];
   float* ys = reinterpret_cast<float*>(lds_raw);
-  __shared__ double s_buf[kNT];
+  __shared__ double s_buf[kLdsMaxNT / 64];
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  lds_stage<float>(L, blk, y, ys);
-  const int lane = threadIdx.x & 63;
+  const LdsWave w = lds_wave(L, blk, n, nslices);
+  const int64_t row = w.pos;
+  SliceHead<uint16_t, HEAD> H;
+  float yi = 0.0f, bv = 0.0f, gv = 0.0f, dv = 0.0f, sv = 0.0f;
+  double rv = 0.0;
+  LdsStage G;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sh);
+  if (w.on) {
+    yi = y[row];
+    bv = ntload(bh + row);
+    gv = ntload(diag + row);
+    if (MODE == kCheb && c1 != 0.0f) dv = ntload(d + row);
+    sv = sd[row];
+    rv = r64[row];
+  }
+  G.finish<float>(L, y, ys);
   double part = 0.0;
-  for (int q = threadIdx.x >> 6; q < L.bs; q += kNT / 64) {
-    const int slice = __builtin_amdgcn_readfirstlane((int)(blk * L.bs + q));
-    if (slice >= nslices) break;
-    const float acc = lds_row_sum<float, uint16_t>(S, L, slice, lane, sh, ys);
-    const int64_t row = (int64_t)slice * 64 + lane;
-    if (row >= n) continue;
-    const float yi = y[row];
-    const float r = ntload(bh + row) - (ntload(diag + row) * yi + acc);
+  float acc = w.on ? lds_row_sum<float>(H, L, w.lane, sh, ys) : float(0);
+  if (w.on) {
+    const float r = bv - (gv * yi + acc);
     float yv;
     if (MODE == kJacobi) {
       yv = yi + c1 * r;
     } else {
-      const float dn = (c1 != 0.0f ? c1 * ntload(d + row) : 0.0f) + c2 * r;
+      const float dn = (c1 != 0.0f ? c1 * dv : 0.0f) + c2 * r;
       yv = yi + dn;
     }
-    const double zv = (double)(sd[row] * yv);
+    const double zv = (double)(sv * yv);
     z[row] = zv;
-    part += r64[row] * zv;
+    part = rv * zv;
   }
-  const double tot = block_sum(part, s_buf);
+  const double tot = block_sum(part, s_buf, blockDim.x >> 6);
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
@@ -562,30 +617,36 @@ __global__ void __launch_bounds__(kNT) pcg_sell_dot_kernel(int64_t n, int64_t ns
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
-// The same on the LDS-staged copy: a block per L.bs slices, p.q partials per block.
-__global__ void __launch_bounds__(kNT) pcg_sell_lds_dot_kernel(int64_t n, int64_t nslices, SellView S, LdsView L,
-                                                             const double* __restrict__ sv,
-                                                             const double* __restrict__ p, double* __restrict__ q,
-                                                             double* __restrict__ partials) {
+// The same on the LDS-staged copy: a block per L.bs slices (a wavefront each),
+// p.q partials per block.
+template <int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) pcg_sell_lds_dot_kernel(
+    int64_t n, int64_t nslices, SellView S, LdsView L, const double* __restrict__ sv, const double* __restrict__ p,
+    double* __restrict__ q, double* __restrict__ partials) {
   extern __shared__ unsigned char lds_raw[];
   double* xs = reinterpret_cast<double*>(lds_raw);
-  __shared__ double s_buf[kNT];
+  __shared__ double s_buf[kLdsMaxNT / 64];
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-  lds_stage<double>(L, blk, p, xs);
-  const int lane = threadIdx.x & 63;
-  double part = 0.0;
-  for (int w = threadIdx.x >> 6; w < L.bs; w += kNT / 64) {
-    const int slice = __builtin_amdgcn_readfirstlane((int)(blk * L.bs + w));
-    if (slice >= nslices) break;
-    double acc = lds_row_sum<double>(S, L, slice, lane, sv, xs);
-    const int64_t row = (int64_t)slice * 64 + lane;
-    if (row < n) {
-      if (S.sd64) acc += S.sd64[row] * p[row];  // the diagonal term, last
-      q[row] = acc;
-      part += acc * p[row];
-    }
+  const LdsWave w = lds_wave(L, blk, n, nslices);
+  const int64_t row = w.pos;
+  SliceHead<double, HEAD> H;
+  double pv = 0.0, sdv = 0.0;
+  LdsStage G;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sv);
+  if (w.on) {
+    pv = p[row];
+    if (S.sd64) sdv = S.sd64[row];
   }
-  double tot = block_sum(part, s_buf);
+  G.finish<double>(L, p, xs);
+  double part = 0.0;
+  double acc = w.on ? lds_row_sum<double>(H, L, w.lane, sv, xs) : double(0);
+  if (w.on) {
+    if (S.sd64) acc += sdv * pv;  // the diagonal term, last
+    q[row] = acc;
+    part = acc * pv;
+  }
+  const double tot = block_sum(part, s_buf, blockDim.x >> 6);
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
@@ -1101,20 +1162,19 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
   };
   auto last_step = [&](int mode, T* cur, double c1, double c2) {
     if (A.lds_bs > 0) {
-      const unsigned nb = (unsigned)((A.nslices + A.lds_bs - 1) / A.lds_bs);
       const size_t lds = sizeof(float) * (size_t)A.lds_maxc;
-      if (mode == kJacobi)
-        sell_lds_out_kernel<kJacobi><<<nb, kNT, lds, s>>>(A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(),
-                                                          (const float*)cur, (const float*)b, (const float*)dinv,
-                                                          (const float*)d, (float)c1, (float)c2, io->r64, io->z64,
-                                                          io->partials);
-      else
-        sell_lds_out_kernel<kCheb><<<nb, kNT, lds, s>>>(A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(),
-                                                        (const float*)cur, (const float*)b, (const float*)dinv,
-                                                        (const float*)d, (float)c1, (float)c2, io->r64, io->z64,
-                                                        io->partials);
+      lds_launch(A, 4, [&](auto head, unsigned nb, unsigned nt) {
+        if (mode == kJacobi)
+          sell_lds_out_kernel<kJacobi, head.value><<<nb, nt, lds, s>>>(
+              A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(), (const float*)cur, (const float*)b,
+              (const float*)dinv, (const float*)d, (float)c1, (float)c2, io->r64, io->z64, io->partials);
+        else
+          sell_lds_out_kernel<kCheb, head.value><<<nb, nt, lds, s>>>(
+              A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(), (const float*)cur, (const float*)b,
+              (const float*)dinv, (const float*)d, (float)c1, (float)c2, io->r64, io->z64, io->partials);
+        io->nb = nb;
+      });
       HIP_LAUNCH_CHECK();
-      io->nb = nb;
       return;
     }
     const unsigned g = grid_for(A.nslices, kNT / 64);
@@ -1326,14 +1386,27 @@ unsigned vcycle0_half(Handle& h, const double* r64, double* z64, double* partial
                                      4.0 * ((double)O.nnz - O.nnz_compact);
   const double step_bytes = mbytes + 4.0 * n * (S.type ? 6.0 : 4.0);
   const bool prof = h.profiling;
+  auto staged_step = [&](auto mode, float c1, float c2) {
+    lds_launch(O, 2, [&](auto head, unsigned nb, unsigned nt) {
+      sell_half_lds_kernel<mode.value, head.value><<<nb, nt, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(),
+                                                                       H.ah_diag.get(), cur, bh, rr, d, nxt, c1, c2);
+    });
+  };
+  auto staged_out = [&](auto mode, float c1, float c2) {
+    lds_launch(O, 2, [&](auto head, unsigned nb, unsigned nt) {
+      sell_half_lds_out_kernel<mode.value, head.value><<<nb, nt, ldsb, s>>>(
+          n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(), H.ah_s.get(), cur, bh, d, c1, c2, r64, z64, partials);
+    });
+  };
+  using ModeResid = std::integral_constant<int, kResid>;
+  using ModeJacobi = std::integral_constant<int, kJacobi>;
+  using ModeCheb = std::integral_constant<int, kCheb>;
   auto step = [&](int mode, double c1, double c2) {
     ProfScope ps(h, prof ? "smooth_l0_h" : "", step_bytes);
     if (staged && mode == kJacobi)
-      sell_half_lds_kernel<kJacobi><<<gl, kNT, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(), cur,
-                                                           bh, nullptr, nullptr, nxt, (float)c1, 0.0f);
+      staged_step(ModeJacobi{}, (float)c1, 0.0f);
     else if (staged)
-      sell_half_lds_kernel<kCheb><<<gl, kNT, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(), cur, bh,
-                                                         nullptr, d, nxt, (float)c1, (float)c2);
+      staged_step(ModeCheb{}, (float)c1, (float)c2);
     else if (mode == kJacobi)
       sell_half_kernel<kJacobi><<<g, kNT, 0, s>>>(n, O.nslices, V, O.sh.get(), H.ah_diag.get(), cur, bh, nullptr,
                                                   nullptr, nxt, (float)c1, 0.0f);
@@ -1355,8 +1428,7 @@ unsigned vcycle0_half(Handle& h, const double* r64, double* z64, double* partial
   }
   // residual, restriction, coarse correction, prolongation
   if (staged)
-    sell_half_lds_kernel<kResid><<<gl, kNT, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(), cur, bh,
-                                                        rr, nullptr, nullptr, 0.0f, 0.0f);
+    staged_step(ModeResid{}, 0.0f, 0.0f);
   else
     sell_half_kernel<kResid><<<g, kNT, 0, s>>>(n, O.nslices, V, O.sh.get(), H.ah_diag.get(), cur, bh, rr, nullptr,
                                                 nullptr, 0.0f, 0.0f);
@@ -1376,13 +1448,9 @@ unsigned vcycle0_half(Handle& h, const double* r64, double* z64, double* partial
     ProfScope ps(h, prof ? "smooth_l0_h_out" : "", step_bytes + 12.0 * n);
     if (staged) {
       if (S.type)
-        sell_half_lds_out_kernel<kCheb><<<gl, kNT, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(),
-                                                               H.ah_s.get(), cur, bh, d, (float)c1, (float)c2, r64,
-                                                               z64, partials);
+        staged_out(ModeCheb{}, (float)c1, (float)c2);
       else
-        sell_half_lds_out_kernel<kJacobi><<<gl, kNT, ldsb, s>>>(n, O.nslices, V, LV_, O.sh.get(), H.ah_diag.get(),
-                                                                 H.ah_s.get(), cur, bh, nullptr, (float)c1, 0.0f,
-                                                                 r64, z64, partials);
+        staged_out(ModeJacobi{}, (float)c1, 0.0f);
       HIP_LAUNCH_CHECK();
       continue;
     }
@@ -1805,11 +1873,14 @@ void launch_sell_dot(Handle& h) {
   if (A.srow.size() || A.sell_g != 1)
     fail(FEM_ERR_STATE, "the operator's sliced-ELL copy must keep the row order with one lane per row");
   if (A.lds_bs > 0) {
-    const unsigned nb = (unsigned)((A.nslices + A.lds_bs - 1) / A.lds_bs);
-    pcg_sell_lds_dot_kernel<<<nb, kNT, sizeof(double) * (size_t)A.lds_maxc, h.stream>>>(
-        A.n, A.nslices, sell_view(A), lds_view(A), A.s64.get(), h.kp.get(), h.kq.get(), h.partials.get());
+    unsigned blocks = 0;
+    lds_launch(A, 8, [&](auto head, unsigned nb, unsigned nt) {
+      pcg_sell_lds_dot_kernel<head.value><<<nb, nt, sizeof(double) * (size_t)A.lds_maxc, h.stream>>>(
+          A.n, A.nslices, sell_view(A), lds_view(A), A.s64.get(), h.kp.get(), h.kq.get(), h.partials.get());
+      blocks = nb;
+    });
     HIP_LAUNCH_CHECK();
-    finish(h, (int)nb, 1, F_ALPHA, 0);
+    finish(h, (int)blocks, 1, F_ALPHA, 0);
     return;
   }
   unsigned g = grid_for(A.nslices, kNT / 64);
