@@ -948,11 +948,8 @@ void sell_or_csr(Csr& M, int64_t sort_window, int lanes, bool with_f32, hipStrea
   M.sd64.release();
   M.sd32.release();
   M.nnz_sdiag = 0;
-  M.lds_bs = 0;
-  M.lds_maxc = 0;
-  M.lc.release();
-  M.lcs.release();
-  M.lcols.release();
+  M.lds.clear();
+  M.ldm.clear();
 }
 
 }  // namespace
@@ -979,7 +976,7 @@ void build_half_level0(Handle& h) {
   HIP_LAUNCH_CHECK();
   build_sell(O, false, s, 0, /*with_f16=*/true, /*with_f64=*/false);
   // y staged in LDS per block of slices, as for the FP32 fine operator
-  build_lds(O, lds_block_slices(O), s);
+  build_lds(O, lds_block_slices(O), O.lds, s);
   O.v64.release();  // only the FP16 sliced copy is used
   // D^1/2 P (sliced ELL, FP32, rows sorted by length) and its transpose (CSR, FP32)
   copy_csr(L0.P, H.ph, s);
@@ -1032,7 +1029,7 @@ void build_hierarchy(Handle& h) {
   // blocks of 8 slices stage their distinct columns of x in LDS (measured at
   // 161^3: 8 slices per block 75 us per FP32 SpMV against 77 with 16 and 94
   // with gathers from memory)
-  build_lds(h.A, lds_block_slices(h.A), s);
+  build_lds(h.A, lds_block_slices(h.A), h.A.lds, s);
 
   int64_t total_rows = 0, total_nnz = 0;
   std::unique_ptr<Level> cur(new Level());
@@ -1186,7 +1183,7 @@ void build_hierarchy(Handle& h) {
     // 18.4 us for the 4-lane copy without staging)
     if (l > 0 && A.n >= kLdsCoarseRows) {
       sell_or_csr(A, 0, 1, H.precision >= 1, s, true);
-      build_lds(A, lds_block_slices(A), s);
+      build_lds(A, lds_block_slices(A), A.lds, s);
     } else if (l > 0) {
       sell_or_csr(A, 0, sell_lanes(A), H.precision >= 1, s);
     }
@@ -1196,7 +1193,7 @@ void build_hierarchy(Handle& h) {
       sell_or_csr(L.P, 1024, sell_lanes(L.P), H.precision >= 1, s);
       // prolongators of many rows: the coarse vector staged in LDS (161^3 level
       // 0: 52.5 -> 41.0 us per prolongation)
-      if (L.P.n >= kLdsCoarseRows) build_lds(L.P, lds_block_slices(L.P), s);
+      if (L.P.n >= kLdsCoarseRows) build_lds(L.P, lds_block_slices(L.P), L.P.lds, s);
       sell_or_csr(L.R, 0, sell_lanes(L.R), H.precision >= 1, s);
     }
   }

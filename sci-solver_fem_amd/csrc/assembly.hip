@@ -713,20 +713,20 @@ __global__ void kappa_gather_kernel(int64_t ne, const int32_t* __restrict__ eper
   if (e < ne) k[e] = ku[eperm[e]];
 }
 
-__global__ void gather_kernel(int64_t n, int k, const int32_t* __restrict__ perm, const double* __restrict__ in,
-                              double* __restrict__ out) {
+__global__ void gather_kernel(int64_t n, int k, int kk, const int32_t* __restrict__ perm,
+                              const double* __restrict__ in, double* __restrict__ out) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * k) return;
-  int64_t i = t / k, c = t - i * k;
-  out[t] = in[(int64_t)perm[i] * k + c];
+  if (t >= n * kk) return;
+  int64_t i = t / kk, c = t - i * kk;
+  out[t] = c < k ? in[(int64_t)perm[i] * k + c] : 0.0;
 }
 
-__global__ void scatter_kernel(int64_t n, int k, const int32_t* __restrict__ perm, const double* __restrict__ in,
-                               double* __restrict__ out) {
+__global__ void scatter_kernel(int64_t n, int k, int kk, const int32_t* __restrict__ perm,
+                               const double* __restrict__ in, double* __restrict__ out) {
   int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n * k) return;
   int64_t i = t / k, c = t - i * k;
-  out[(int64_t)perm[i] * k + c] = in[t];
+  out[(int64_t)perm[i] * k + c] = in[i * kk + c];
 }
 
 // bit 0: a vertex index outside [0, nv); bit 1: NaN coefficient; bit 2: NaN coordinate
@@ -1051,15 +1051,15 @@ void set_kappa_user(Handle& h, const double* kappa_user_dev) {
   HIP_LAUNCH_CHECK();
 }
 
-void gather_user_to_int(Handle& h, const double* u, double* i, int k) {
+void gather_user_to_int(Handle& h, const double* u, double* i, int k, int kk) {
   int64_t n = h.A.n;
-  gather_kernel<<<grid_for(n * k, 256), 256, 0, h.stream>>>(n, k, h.perm.get(), u, i);
+  gather_kernel<<<grid_for(n * kk, 256), 256, 0, h.stream>>>(n, k, kk, h.perm.get(), u, i);
   HIP_LAUNCH_CHECK();
 }
 
-void scatter_int_to_user(Handle& h, const double* i, double* u, int k) {
+void scatter_int_to_user(Handle& h, const double* i, double* u, int k, int kk) {
   int64_t n = h.A.n;
-  scatter_kernel<<<grid_for(n * k, 256), 256, 0, h.stream>>>(n, k, h.perm.get(), i, u);
+  scatter_kernel<<<grid_for(n * k, 256), 256, 0, h.stream>>>(n, k, kk, h.perm.get(), i, u);
   HIP_LAUNCH_CHECK();
 }
 

@@ -176,23 +176,24 @@ void ensure_setup(Handle& h) {
   }
 }
 
-// stage nv x k user-order data into internal order on the device
-void to_internal(Handle& h, const double* src, int on_device, double* dst, int k) {
+// stage nv x k user-order data into internal order on the device (rows of kk
+// >= k columns, the others zero)
+void to_internal(Handle& h, const double* src, int on_device, double* dst, int k, int kk) {
   const int64_t m = h.A.n * k;
   const double* dsrc = src;
   if (!on_device) {
     HIP_CHECK(hipMemcpyAsync(h.ubuf.get(), src, sizeof(double) * m, hipMemcpyHostToDevice, h.stream));
     dsrc = h.ubuf.get();
   }
-  gather_user_to_int(h, dsrc, dst, k);
+  gather_user_to_int(h, dsrc, dst, k, kk);
 }
 
-void from_internal(Handle& h, const double* src, double* dst, int on_device, int k) {
+void from_internal(Handle& h, const double* src, double* dst, int on_device, int k, int kk) {
   const int64_t m = h.A.n * k;
   if (on_device) {
-    scatter_int_to_user(h, src, dst, k);
+    scatter_int_to_user(h, src, dst, k, kk);
   } else {
-    scatter_int_to_user(h, src, h.ubuf2.get(), k);
+    scatter_int_to_user(h, src, h.ubuf2.get(), k, kk);
     HIP_CHECK(hipMemcpyAsync(dst, h.ubuf2.get(), sizeof(double) * m, hipMemcpyDeviceToHost, h.stream));
   }
   HIP_CHECK(hipStreamSynchronize(h.stream));
@@ -470,11 +471,12 @@ int fem_solve(fem_handle* hh, const double* b, double* x, int nrhs, int on_devic
       ensure_setup(h);
       setup_ms = h.H.setup_ms;
     }
-    ensure_krylov(h, nrhs);
-    to_internal(h, b, on_device, h.kb.get(), nrhs);
-    to_internal(h, x, on_device, h.kx.get(), nrhs);
-    int st = pcg_solve(h, nrhs, info);
-    from_internal(h, h.kx.get(), x, on_device, nrhs);
+    const int kk = padded_columns(h, nrhs);
+    ensure_krylov(h, kk);
+    to_internal(h, b, on_device, h.kb.get(), nrhs, kk);
+    to_internal(h, x, on_device, h.kx.get(), nrhs, kk);
+    int st = pcg_solve(h, kk, info);
+    from_internal(h, h.kx.get(), x, on_device, nrhs, kk);
     fill_info(h, info, setup_ms);
     if (st == FEM_ERR_NOT_CONVERGED) h.err = "solve reached maxIters above tolerance";
     return st;
@@ -495,11 +497,11 @@ int fem_adjoint_grad(fem_handle* hh, const double* u, const double* dLdu, double
     }
     ensure_krylov(h, 1);
     // K lambda = dL/du (K symmetric), zero initial guess
-    to_internal(h, dLdu, on_device, h.kb.get(), 1);
+    to_internal(h, dLdu, on_device, h.kb.get(), 1, 1);
     HIP_CHECK(hipMemsetAsync(h.kx.get(), 0, sizeof(double) * h.A.n, h.stream));
     int st = pcg_solve(h, 1, info);
     // u into internal order (kz is free after the solve)
-    to_internal(h, u, on_device, h.kz.get(), 1);
+    to_internal(h, u, on_device, h.kz.get(), 1, 1);
     double* g = dLdkappa;
     DevBuf<double> gdev;
     if (!on_device) {
@@ -510,7 +512,7 @@ int fem_adjoint_grad(fem_handle* hh, const double* u, const double* dLdu, double
     if (!on_device) {
       HIP_CHECK(hipMemcpyAsync(dLdkappa, g, sizeof(double) * h.ne, hipMemcpyDeviceToHost, h.stream));
     }
-    if (lambda_out) from_internal(h, h.kx.get(), lambda_out, on_device, 1);
+    if (lambda_out) from_internal(h, h.kx.get(), lambda_out, on_device, 1, 1);
     HIP_CHECK(hipStreamSynchronize(h.stream));
     fill_info(h, info, setup_ms);
     return st;
@@ -523,8 +525,8 @@ int fem_element_grad(fem_handle* hh, const double* a, const double* u, double* d
     Handle& h = *H(hh);
     if (!h.has_mesh) fail(FEM_ERR_STATE, "no mesh");
     ensure_krylov(h, 1);
-    to_internal(h, a, on_device, h.kq.get(), 1);
-    to_internal(h, u, on_device, h.kz.get(), 1);
+    to_internal(h, a, on_device, h.kq.get(), 1, 1);
+    to_internal(h, u, on_device, h.kz.get(), 1, 1);
     double* g = dLdkappa;
     DevBuf<double> gdev;
     if (!on_device) {
@@ -543,10 +545,11 @@ int fem_apply_operator(fem_handle* hh, const double* x, double* y, int nrhs, int
   return guarded(hh, [&]() {
     Handle& h = *H(hh);
     if (h.A.n == 0) fail(FEM_ERR_EMPTY, "Error no matrix specified");
-    ensure_krylov(h, nrhs);
-    to_internal(h, x, on_device, h.kp.get(), nrhs);
-    apply_operator_int(h, h.kp.get(), h.kq.get(), nrhs);
-    from_internal(h, h.kq.get(), y, on_device, nrhs);
+    const int kk = padded_columns(h, nrhs);
+    ensure_krylov(h, kk);
+    to_internal(h, x, on_device, h.kp.get(), nrhs, kk);
+    apply_operator_int(h, h.kp.get(), h.kq.get(), kk);
+    from_internal(h, h.kq.get(), y, on_device, nrhs, kk);
     return (int)FEM_OK;
   });
 }
@@ -557,9 +560,9 @@ int fem_apply_preconditioner(fem_handle* hh, const double* r, double* z, int on_
     Handle& h = *H(hh);
     ensure_setup(h);
     ensure_krylov(h, 1);
-    to_internal(h, r, on_device, h.kr.get(), 1);
+    to_internal(h, r, on_device, h.kr.get(), 1, 1);
     apply_vcycle_fp64(h, h.kr.get(), h.kz.get());
-    from_internal(h, h.kz.get(), z, on_device, 1);
+    from_internal(h, h.kz.get(), z, on_device, 1, 1);
     return (int)FEM_OK;
   });
 }

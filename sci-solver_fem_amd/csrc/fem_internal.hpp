@@ -24,6 +24,18 @@ namespace fem {
 constexpr int kSellWindows = 8;
 constexpr int kSellWinBits = 13;
 
+// LDS staging lists of a sliced copy: block b of bs consecutive slices copies
+// x at its distinct columns lcols[lcs[b] .. lcs[b+1]) (ascending) into LDS;
+// lc holds each stored entry's 16-bit index into that list (same layout as
+// the copy's columns).  bs == 0: none.
+struct LdsList {
+  int bs = 0;
+  int maxc = 0;  // largest distinct-column count of a block
+  DevBuf<uint16_t> lc;
+  DevBuf<int32_t> lcs, lcols;
+  void clear() { *this = LdsList(); }
+};
+
 // Compressed sparse rows on the device.
 struct Csr {
   int64_t n = 0;    // rows
@@ -61,14 +73,10 @@ struct Csr {
   DevBuf<double> sd64;
   DevBuf<float> sd32;
   int64_t nnz_sdiag = 0;  // diagonal entries held in sd64 / sd32
-  // LDS staging of the gathered vector (one lane per row, row order): block b
-  // of lds_bs consecutive slices first copies x at its distinct columns
-  // lcols[lcs[b] .. lcs[b+1]) (ascending) into LDS; lc holds each stored
-  // entry's 16-bit index into that list (same layout as sc).  lds_bs == 0: none.
-  int lds_bs = 0;
-  int lds_maxc = 0;            // largest distinct-column count of a block
-  DevBuf<uint16_t> lc;
-  DevBuf<int32_t> lcs, lcols;
+  // LDS staging of the gathered vector (one lane per row): lds for one
+  // column; ldm for several columns, where lds has larger blocks than those
+  // kernels take (built by the first solve with several columns)
+  LdsList lds, ldm;
 };
 
 struct Level {
@@ -211,14 +219,15 @@ int check_mesh_device(int64_t nconn, const int32_t* conn, int64_t nv, int64_t ne
                       const double* xyz, hipStream_t s);
 void assemble_values(Handle& h);            // values only, pattern fixed
 void element_gradient(Handle& h, const double* a_int, const double* u_int, double* g_user);
-void gather_user_to_int(Handle& h, const double* u, double* i, int k);   // i[r] = u[perm[r]]
+// i[r] = u[perm[r]]: k user columns in rows of kk >= k internal ones, the others zero
+void gather_user_to_int(Handle& h, const double* u, double* i, int k, int kk);
 // z = M r (user numbering, device pointers) through the static device scratch
 // in solve.hip: no device allocation; needs a built hierarchy and work vectors
 void apply_preconditioner_noalloc(Handle& h, const double* r_user, double* z_user);
 int64_t noalloc_max_rows();
 // resolves the scratch address of the handle's device when it is current
 void noalloc_init(const Handle& h);
-void scatter_int_to_user(Handle& h, const double* i, double* u, int k);  // u[perm[r]] = i[r]
+void scatter_int_to_user(Handle& h, const double* i, double* u, int k, int kk);  // u[perm[r]] = i[r]
 
 // ---- sparse building blocks (sparse.hip) ----
 // C = L * Rm with optional column map on Rm's columns and optional removal of
@@ -233,10 +242,10 @@ void csr_transpose(const Csr& P, Csr& R, hipStream_t s);
 // (square A, one lane per row, row order) keeps the diagonal outside the slices
 void build_sell(Csr& A, bool with_f32, hipStream_t s, int64_t sort_window = 0, bool with_f16 = false,
                 bool with_f64 = true, int lanes = 1, bool split_diag = false);
-// LDS staging lists for A's sliced copy (blocks of bs slices); leaves A
-// unstaged (lds_bs = 0) when a block holds more than 16384 stored entries or
-// more than 8192 distinct columns
-void build_lds(Csr& A, int bs, hipStream_t s);
+// LDS staging lists for A's sliced copy (blocks of bs slices) into out (A.lds
+// or A.ldm); leaves it empty (bs = 0) when a block holds more than 8192
+// distinct columns
+void build_lds(const Csr& A, int bs, LdsList& out, hipStream_t s);
 void spmv64(const Csr& A, const double* x, double* y, hipStream_t s);
 
 // ---- AMG setup (amg_setup.hip) ----
@@ -256,7 +265,10 @@ void aggregate_graph(int64_t n, const int32_t* adj_ptr, const int32_t* adj, int 
                      hipStream_t s);
 
 // ---- solve (solve.hip) ----
-void ensure_krylov(Handle& h, int k);
+// columns the kernels hold for k right-hand sides: k padded with zero columns
+// (a zero right-hand side starts, and stays, converged)
+int padded_columns(const Handle& h, int k);
+void ensure_krylov(Handle& h, int k);  // k padded
 int pcg_solve(Handle& h, int k, fem_solve_info* info);   // uses h.kb (rhs), h.kx (x0 / out), internal order
 void apply_vcycle_fp64(Handle& h, const double* r, double* z);  // level-0 preconditioner, 1 column
 void apply_operator_int(Handle& h, const double* x, double* y, int k);

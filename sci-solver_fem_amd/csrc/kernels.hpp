@@ -173,38 +173,6 @@ __global__ void __launch_bounds__(kNT) csr_vec_kernel(int64_t n, const int32_t* 
   if (lane == 0) spmv_epilogue<MODE, T, V>(row, row, acc, y, x, b, dinv, d, xn, c1, c2);
 }
 
-// k right-hand sides: KP lanes per row (KP = power of two >= k), lane c owns
-// column c and walks the row sequentially.
-template <typename V, typename T, int KP, int MODE>
-__global__ void __launch_bounds__(kNT) csr_multi_kernel(int64_t n, int k, const int32_t* __restrict__ rp,
-                                                      const int32_t* __restrict__ ci, const V* __restrict__ val,
-                                                      const T* __restrict__ x, T* __restrict__ y,
-                                                      const T* __restrict__ b, const V* __restrict__ dinv,
-                                                      T* __restrict__ d, T* __restrict__ xn, T c1, T c2) {
-  const int64_t row = ((int64_t)xcd_block(blockIdx.x, gridDim.x) * kNT + threadIdx.x) / KP;
-  const int c = threadIdx.x & (KP - 1);
-  if (row >= n || c >= k) return;
-  const int s = rp[row], e = rp[row + 1];
-  T acc = T(0);
-  // plain loads: the KP lanes of a row walk its entries one by one, so each
-  // cache line of val / ci is used over several iterations (a nontemporal
-  // hint would evict it after the first).  Four entries per step keep four
-  // independent gathers in flight; the sum stays in entry order.
-  int q = s;
-  for (; q + 4 <= e; q += 4) {
-    const int c0 = ci[q], c1i = ci[q + 1], c2i = ci[q + 2], c3 = ci[q + 3];
-    const T v0 = (T)val[q], v1 = (T)val[q + 1], v2 = (T)val[q + 2], v3 = (T)val[q + 3];
-    const T g0 = x[(int64_t)c0 * k + c], g1 = x[(int64_t)c1i * k + c], g2 = x[(int64_t)c2i * k + c],
-            g3 = x[(int64_t)c3 * k + c];
-    acc += v0 * g0;
-    acc += v1 * g1;
-    acc += v2 * g2;
-    acc += v3 * g3;
-  }
-  for (; q < e; ++q) acc += (T)val[q] * x[(int64_t)ci[q] * k + c];
-  spmv_epilogue<MODE, T, V>(row * k + c, row, acc, y, x, b, dinv, d, xn, c1, c2);
-}
-
 // Sliced ELL, one RHS: a wavefront owns a slice of 64 rows, lane = row; the
 // slice is column-major so every step k is one coalesced 64-wide load of
 // values and of columns, and the k steps are independent loads the compiler
@@ -318,7 +286,7 @@ struct LdsView {
   const int32_t* lcols;  // distinct columns per block, ascending
 };
 
-inline LdsView lds_view(const Csr& A) { return LdsView{A.lds_bs, A.lc.get(), A.lcs.get(), A.lcols.get()}; }
+inline LdsView lds_view(const LdsList& l) { return LdsView{l.bs, l.lc.get(), l.lcs.get(), l.lcols.get()}; }
 
 // x at the block's distinct columns into xs (then a block barrier), in two
 // halves: the first kStageCols columns of each thread are loaded by begin(),
@@ -524,7 +492,6 @@ __global__ void __launch_bounds__(kNT) sell_kernel(int64_t n, int64_t nslices, S
 // k right-hand sides with k a multiple of VW = 16 / sizeof(T): L lanes per
 // row, each lane owns VW consecutive columns and gathers them as one 16-byte
 // load (measured for k = 16 FP32 at 161^3: 1.6x the one-column-per-lane kernel).
-// Same per-column summation order as csr_multi_kernel.
 template <typename T, int L, int MODE>
 __global__ void __launch_bounds__(kNT) csr_multi_vec_kernel(int64_t n, int k, const int32_t* __restrict__ rp,
                                                           const int32_t* __restrict__ ci, const T* __restrict__ val,
@@ -725,6 +692,180 @@ __global__ void __launch_bounds__(kNT) sell_multi_kernel(int64_t n, int k, int64
   }
 }
 
+// ---- k right-hand sides on the LDS-staged copy ------------------------------------
+// A block of L.bs slices takes the columns in chunks of VW * LN: it stages x's
+// rows at its distinct columns (one gather of VW * LN values per listed
+// column, 3.4 of them per row at 161^3 against 14 entries), then LN lanes per
+// row, VW consecutive columns each, read the entries' x rows from LDS.  With x
+// gathered per entry the address unit bounded the pass.  What bounds it now is
+// the chain list -> columns -> x -> LDS -> row vectors of each block, hidden
+// only by other wavefronts: full occupancy (at most 64 registers) beats loads
+// issued ahead (161^3, 16 columns, FP32 step 479 us unstaged, 417 staged; 476
+// with the row's vectors and entries loaded before the staging at 5 wavefronts
+// a SIMD).  FP64 rows of 16 columns have eight lanes; there the lanes of a
+// quad load one entry each of four and share them by DPP (operator + p.q 738
+// us unstaged, 747 staged with all lanes loading every code and value, the
+// address unit 70 % busy, 721 shared).  61 x 58 x 73, 5 columns in 8, FP64
+// step: 39.8 us with a lane per column on the CSR arrays, 23.2 us.
+// Per column the sum is in entry order, as in sell_multi_kernel.  DOT 1:
+// per-block, per-column partials of x.y (the operator's p.q); DOT 2: of r.xn
+// (the last smoothing step's r.z).
+template <typename T, int VW>
+struct VecOf {
+  typedef T type __attribute__((ext_vector_type(VW)));
+};
+
+// v of lane J of each quad
+template <int J>
+__device__ __forceinline__ int quad_bcast(int v) {
+  return __builtin_amdgcn_mov_dpp(v, J * 0x55, 0xf, 0xf, true);
+}
+template <int J>
+__device__ __forceinline__ double quad_bcast(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint64_t lo = (uint32_t)quad_bcast<J>((int)(uint32_t)u), hi = (uint32_t)quad_bcast<J>((int)(uint32_t)(u >> 32));
+  return __builtin_bit_cast(double, hi << 32 | lo);
+}
+
+// acc += v_j * x row of entry j, j = 0..3 of the quad's four entries (m of them real)
+template <typename T, typename Vec>
+__device__ __forceinline__ void quad_entries(int c, T v, int m, const Vec* xl, int stride, Vec& acc) {
+  acc += quad_bcast<0>(v) * xl[quad_bcast<0>(c) * stride];
+  if (m > 1) acc += quad_bcast<1>(v) * xl[quad_bcast<1>(c) * stride];
+  if (m > 2) acc += quad_bcast<2>(v) * xl[quad_bcast<2>(c) * stride];
+  if (m > 3) acc += quad_bcast<3>(v) * xl[quad_bcast<3>(c) * stride];
+}
+
+// the row's sum over its w entries; cp, vp: the row's first code and value,
+// xl: this lane's piece of the staged rows
+template <typename T, int LN, typename Vec>
+__device__ __forceinline__ Vec multi_row_sum(const uint16_t* cp, const T* vp, int w, const Vec* xl) {
+  Vec acc = (Vec)(T(0));
+  if constexpr (sizeof(T) == 8) {
+    const int q4 = threadIdx.x & 3;  // entry 4 g + q4 of the row is this lane's of group g
+    for (int g = 0; 4 * g < w; ++g) {
+      int ec = 0;
+      T ev = T(0);
+      if (4 * g + q4 < w) {
+        ec = cp[64 * (4 * g + q4)];
+        ev = vp[64 * (4 * g + q4)];
+      }
+      quad_entries(ec, ev, w - 4 * g, xl, LN, acc);
+    }
+  } else {
+    int q = 0;
+    for (; q + 4 <= w; q += 4) {
+      unsigned i[4];
+      T v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        i[j] = cp[64 * (q + j)];
+        v[j] = vp[64 * (q + j)];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc += v[j] * xl[i[j] * LN];
+    }
+    for (; q < w; ++q) acc += vp[64 * q] * xl[cp[64 * q] * LN];
+  }
+  return acc;
+}
+
+constexpr int kMultiSlices = 2;  // slices per block at most
+
+template <typename T, int VW, int LN, int MODE, int DOT>
+__global__ void __launch_bounds__(64 * kMultiSlices * LN, 8) sell_lds_multi_kernel(
+    int64_t n, int k, int64_t nslices, SellView S, LdsView L, const T* __restrict__ sv, const T* __restrict__ x,
+    T* __restrict__ y, const T* __restrict__ b, const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ xn,
+    T c1, T c2, const double* __restrict__ r64, double* __restrict__ partials) {
+  typedef typename VecOf<T, VW>::type vec;
+  static_assert(LN >= 4 && 64 % LN == 0, "whole quads per row, rows of one slice per wavefront");
+  extern __shared__ unsigned char lds_raw[];
+  vec* xs = reinterpret_cast<vec*>(lds_raw);
+  __shared__ double s_dot[DOT ? kMultiSlices * LN * VW * LN : 1];
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int lc0 = L.lcs[blk], npiece = (L.lcs[blk + 1] - lc0) * LN;
+  const int rl = tid / LN, piece = tid % LN;
+  const int slice = __builtin_amdgcn_readfirstlane((int)blk * L.bs + (rl >> 6));
+  const int64_t pos = (int64_t)slice * 64 + (rl & 63);
+  const bool on = slice < nslices && pos < n;  // the same for the lanes of a row
+  int off = 0, w = 0;
+  if (slice < nslices) {
+    off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
+    w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - off) >> 6);
+  }
+  const T* vp = sv + off + (rl & 63);
+  const uint16_t* cp = L.lc + off + (rl & 63);
+  int64_t row = pos;
+  if (on && S.srow) row = S.srow[pos];
+  const T* sdp = sell_diag<T>(S);
+  for (int cb = 0; cb < k; cb += VW * LN) {
+    if (cb) __syncthreads();  // the previous chunk's LDS rows are read
+    for (int t = tid; t < npiece; t += nt) {
+      const int c = cb + (t % LN) * VW;
+      if (c < k) xs[t] = *(const vec*)(x + (int64_t)L.lcols[lc0 + t / LN] * k + c);
+    }
+    __syncthreads();
+    const int c = cb + piece * VW;
+    double part[VW];
+#pragma unroll
+    for (int j = 0; j < VW; ++j) part[j] = 0.0;
+    if (on) {
+      vec acc = multi_row_sum<T, LN>(cp, vp, w, xs + piece);
+      if (c < k) {
+        const int64_t idx = row * k + c;
+        vec xv = (vec)(T(0));
+        if (sdp || MODE == kJacobi || MODE == kCheb || DOT == 1) xv = *(const vec*)(x + idx);
+        if (sdp) acc += sdp[row] * xv;  // the diagonal term, last
+        vec out = acc;
+        if (MODE == kAssign) {
+          *(vec*)(y + idx) = acc;
+        } else if (MODE == kAssignScale) {
+          *(vec*)(y + idx) = acc;
+          out = (c1 * dinv[row]) * acc;
+          *(vec*)(xn + idx) = out;
+          if (d) *(vec*)(d + idx) = out;
+        } else if (MODE == kResid) {
+          *(vec*)(y + idx) = *(const vec*)(b + idx) - acc;
+        } else if (MODE == kAdd) {
+          *(vec*)(y + idx) += acc;
+        } else if (MODE == kJacobi) {
+          out = xv + (c1 * dinv[row]) * (*(const vec*)(b + idx) - acc);
+          *(vec*)(xn + idx) = out;
+        } else {  // kCheb (d is not needed after a last step, DOT 2)
+          const vec r = dinv[row] * (*(const vec*)(b + idx) - acc);
+          const vec dn = (c1 != T(0) ? c1 * *(const vec*)(d + idx) : (vec)(T(0))) + c2 * r;
+          if (DOT != 2) *(vec*)(d + idx) = dn;
+          out = xv + dn;
+          *(vec*)(xn + idx) = out;
+        }
+        if (DOT == 1) {
+#pragma unroll
+          for (int j = 0; j < VW; ++j) part[j] = (double)xv[j] * (double)acc[j];
+        } else if (DOT == 2) {
+#pragma unroll
+          for (int j = 0; j < VW; ++j) part[j] = r64[idx + j] * (double)out[j];
+        }
+      }
+    }
+    if (DOT) {
+      // over the wavefront's rows, then over the wavefronts (fixed order)
+#pragma unroll
+      for (int j = 0; j < VW; ++j) {
+#pragma unroll
+        for (int o = 32; o >= LN; o >>= 1) part[j] += __shfl_xor(part[j], o, 64);
+        if ((tid & 63) < LN) s_dot[((tid >> 6) * LN + piece) * VW + j] = part[j];
+      }
+      __syncthreads();
+      if (tid < VW * LN && cb + tid < k) {
+        double t = 0.0;
+        for (int i = 0; i < (nt >> 6); ++i) t += s_dot[i * VW * LN + tid];
+        partials[(int64_t)(cb + tid) * gridDim.x + blockIdx.x] = t;
+      }
+    }
+  }
+}
+
 // ---- reductions ---------------------------------------------------------------
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -748,7 +889,8 @@ __device__ __forceinline__ double block_sum(double v, double* s_buf, int waves =
 }
 
 // Per-column block partials for row-major (n x k) data: thread (row, c) with
-// c = tid % KP.  Writes partials[blockIdx.x * k + c] for c < k.
+// c = tid % KP.  Writes partials[c * gridDim.x + blockIdx.x] for c < k (a
+// column's partials are consecutive for the finish).
 template <int KP>
 __device__ __forceinline__ void block_col_partials(double v, int k, double* s_buf, double* partials) {
   if (KP == 1) {
@@ -761,7 +903,7 @@ __device__ __forceinline__ void block_col_partials(double v, int k, double* s_bu
   if ((int)threadIdx.x < k) {
     double s = 0.0;
     for (int j = threadIdx.x; j < kNT; j += KP) s += s_buf[j];
-    partials[(int64_t)blockIdx.x * k + threadIdx.x] = s;
+    partials[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
   }
   __syncthreads();
 }

@@ -128,14 +128,6 @@ void launch_multi_vec(const Csr& A, int k, const T* val, const T* x, T* y, const
                                                         c1, c2);
 }
 
-template <typename V, typename T, int MODE, int KP>
-void launch_multi(const Csr& A, int k, const V* val, const T* x, T* y, const T* b, const V* dinv, T* d, T* xn, T c1,
-                  T c2, hipStream_t s) {
-  unsigned grid = grid_for(A.n * KP, kNT);
-  csr_multi_kernel<V, T, KP, MODE><<<grid, kNT, 0, s>>>(A.n, k, A.rp.get(), A.ci.get(), val, x, y, b, dinv, d, xn,
-                                                       c1, c2);
-}
-
 template <typename T>
 const T* svals_of(const Csr& A);
 template <>
@@ -187,17 +179,70 @@ constexpr int64_t kLdsHeadRow = 20;  // average row length above which no head i
 //    code of the head costs more than it hides (3.25 us against 3.6).
 template <typename Fn>
 void lds_launch(const Csr& A, size_t vsize, Fn&& f) {
-  const unsigned nb = (unsigned)((A.nslices + A.lds_bs - 1) / A.lds_bs);
-  const unsigned nt = 64u * (unsigned)A.lds_bs;
+  const unsigned nb = (unsigned)((A.nslices + A.lds.bs - 1) / A.lds.bs);
+  const unsigned nt = 64u * (unsigned)A.lds.bs;
   const bool lengths = A.srow.size() > 0;  // rows in length order (prolongators)
   if (nb < 256u || A.nnz > kLdsHeadRow * A.n)
     f(std::integral_constant<int, 0>{}, nb, nt < 256u ? 256u : nt);
-  else if (A.lds_bs > 2 && vsize == 8)
+  else if (A.lds.bs > 2 && vsize == 8)
     f(std::integral_constant<int, 0>{}, nb, nt);
   else if (A.nnz <= 8 * A.n && !lengths)
     f(std::integral_constant<int, 8>{}, nb, nt);
   else
     f(std::integral_constant<int, kLdsHead>{}, nb, nt);
+}
+
+// ---- several columns on the staged copy
+constexpr int kMultiLds = 122880;  // bytes of x rows a block stages at most
+
+const LdsList& multi_list(const Csr& A) { return A.ldm.bs > 0 ? A.ldm : A.lds; }
+
+// columns per lane and lanes per row: 16 FP32 columns by four lanes, 16 FP64
+// columns by eight (16 bytes a lane); 4 or 8 columns by four lanes.  Operators
+// with a staged copy take it whatever their row length (161^3 level 1, ~46
+// entries: 43.9 us a step against 52.2 for the entry-split CSR kernel)
+template <typename T>
+int multi_cols(int k) { return std::min(pow2_at_least(k / 4), 16 / (int)sizeof(T)); }
+template <typename T>
+int multi_lanes(int k) { return sizeof(T) == 8 && k > 8 ? 8 : 4; }
+
+template <typename T>
+size_t multi_lds(const Csr& A, int k) {
+  return (size_t)multi_list(A).maxc * multi_cols<T>(k) * multi_lanes<T>(k) * sizeof(T);
+}
+
+template <typename T>
+bool multi_staged(const Csr& A, int k) {
+  const LdsList& M = multi_list(A);
+  return k > 1 && k % 4 == 0 && A.nslices > 0 && A.sell_g == 1 && svals_of<T>(A) && M.bs > 0 &&
+         M.bs <= kMultiSlices && multi_lds<T>(A, k) <= (size_t)kMultiLds;
+}
+
+unsigned multi_blocks(const Csr& A) { return (unsigned)((A.nslices + multi_list(A).bs - 1) / multi_list(A).bs); }
+
+template <typename T, int MODE, int DOT>
+void launch_lds_multi(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T* d, T* xn, T c1, T c2,
+                      const double* r64, double* partials, hipStream_t s) {
+  const LdsList& M = multi_list(A);
+  auto go = [&](auto vw, auto ln) {
+    constexpr int VW = decltype(vw)::value, LN = decltype(ln)::value;
+    sell_lds_multi_kernel<T, VW, LN, MODE, DOT><<<multi_blocks(A), 64 * M.bs * LN, multi_lds<T>(A, k), s>>>(
+        A.n, k, A.nslices, sell_view(A), lds_view(M), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2, r64, partials);
+  };
+  using One = std::integral_constant<int, 1>;
+  using Two = std::integral_constant<int, 2>;
+  using Four = std::integral_constant<int, 4>;
+  using Eight = std::integral_constant<int, 8>;
+  const int vw = multi_cols<T>(k);
+  if (vw == 1)
+    go(One{}, Four{});
+  else if constexpr (sizeof(T) == 8) {
+    if (multi_lanes<T>(k) == 4) go(Two{}, Four{});
+    else go(Two{}, Eight{});
+  } else {
+    if (vw == 2) go(Two{}, Four{});
+    else go(Four{}, Four{});
+  }
 }
 
 // y/xn = f(A x) for k right-hand sides; MODE selects the epilogue.  One RHS
@@ -207,10 +252,10 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
              hipStream_t s) {
   if (A.n == 0) return;
   const T* val = vals_of<T>(A);
-  if (k == 1 && A.nslices > 0 && svals_of<T>(A) && A.lds_bs > 0) {
+  if (k == 1 && A.nslices > 0 && svals_of<T>(A) && A.lds.bs > 0) {
     lds_launch(A, sizeof(T), [&](auto head, unsigned nb, unsigned nt) {
-      sell_lds_kernel<T, MODE, head.value><<<nb, nt, sizeof(T) * (size_t)A.lds_maxc, s>>>(
-          A.n, A.nslices, sell_view(A), lds_view(A), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2);
+      sell_lds_kernel<T, MODE, head.value><<<nb, nt, sizeof(T) * (size_t)A.lds.maxc, s>>>(
+          A.n, A.nslices, sell_view(A), lds_view(A.lds), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2);
     });
   } else if (k == 1 && A.nslices > 0 && svals_of<T>(A)) {
     switch (A.sell_g) {
@@ -229,6 +274,8 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
       case 32: launch_vec<T, T, MODE, 32>(A, val, x, y, b, dinv, d, xn, c1, c2, s); break;
       default: launch_vec<T, T, MODE, 64>(A, val, x, y, b, dinv, d, xn, c1, c2, s); break;
     }
+  } else if (MODE != kAdd && multi_staged<T>(A, k)) {  // prolongators: short rows, 196 us unstaged, 202 staged
+    launch_lds_multi<T, MODE, 0>(A, k, x, y, b, dinv, d, xn, c1, c2, nullptr, nullptr, s);
   } else if (k % sell_multi_cols<T>() == 0 && A.nslices > 0 && A.sell_g == 1 && svals_of<T>(A) &&
              A.nnz <= kMultiSellRow * A.n) {
     // column groups on the sliced-ELL copy
@@ -240,8 +287,10 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
       case 16: launch_sell_multi<T, MODE, 16>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
       default: launch_sell_multi<T, MODE, 32>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
     }
-  } else if (k % (16 / (int)sizeof(T)) == 0) {
-    // 16-byte column groups (all multi-column vectors here come from hipMalloc)
+  } else {
+    // 16-byte column groups (all multi-column vectors here come from hipMalloc;
+    // padded_columns keeps k a multiple of the group)
+    if (k % (16 / (int)sizeof(T)) != 0) fail(FEM_ERR_STATE, "column count is not padded");
     switch (pow2_at_least(k / (16 / (int)sizeof(T)))) {
       case 1: launch_multi_vec<T, MODE, 1>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
       case 2: launch_multi_vec<T, MODE, 2>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
@@ -249,15 +298,6 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
       case 8: launch_multi_vec<T, MODE, 8>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
       case 16: launch_multi_vec<T, MODE, 16>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
       default: launch_multi_vec<T, MODE, 32>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-    }
-  } else {
-    switch (pow2_at_least(k)) {
-      case 2: launch_multi<T, T, MODE, 2>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-      case 4: launch_multi<T, T, MODE, 4>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-      case 8: launch_multi<T, T, MODE, 8>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-      case 16: launch_multi<T, T, MODE, 16>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-      case 32: launch_multi<T, T, MODE, 32>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
-      default: launch_multi<T, T, MODE, 64>(A, k, val, x, y, b, dinv, d, xn, c1, c2, s); break;
     }
   }
   HIP_LAUNCH_CHECK();
@@ -650,38 +690,6 @@ __global__ void __launch_bounds__(kLdsMaxNT) pcg_sell_lds_dot_kernel(
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
-// q = A p and per-block, per-column partials of p.q (k columns)
-template <int KP>
-__global__ void __launch_bounds__(kNT) pcg_spmm_dot_kernel(int64_t n, int k, const int32_t* __restrict__ rp,
-                                                         const int32_t* __restrict__ ci,
-                                                         const double* __restrict__ val, const double* __restrict__ p,
-                                                         double* __restrict__ q, double* __restrict__ partials) {
-  __shared__ double s_buf[kNT];
-  double part = 0.0;
-  const int c = threadIdx.x & (KP - 1);
-  // kNT / KP rows per pass, one front per XCD
-  const XcdRows R = xcd_rows(n, kNT / KP);
-  if (c < k) {
-    for (int64_t row = R.first + threadIdx.x / KP; row < R.hi; row += R.step) {
-      const int s = rp[row], e = rp[row + 1];
-      double acc = 0.0;
-      int j = s;
-      for (; j + 4 <= e; j += 4) {
-        const double g0 = p[(int64_t)ci[j] * k + c], g1 = p[(int64_t)ci[j + 1] * k + c],
-                     g2 = p[(int64_t)ci[j + 2] * k + c], g3 = p[(int64_t)ci[j + 3] * k + c];
-        acc += val[j] * g0;
-        acc += val[j + 1] * g1;
-        acc += val[j + 2] * g2;
-        acc += val[j + 3] * g3;
-      }
-      for (; j < e; ++j) acc += val[j] * p[(int64_t)ci[j] * k + c];
-      q[row * k + c] = acc;
-      part += acc * p[row * k + c];
-    }
-  }
-  block_col_partials<KP>(part, k, s_buf, partials);
-}
-
 // x += alpha p; r -= alpha q; partials of r.r
 // (and r32 = fl32(r), the FP32 V-cycle's input, when r32 is given)
 template <int KP>
@@ -717,8 +725,9 @@ __global__ void __launch_bounds__(kNT) pcg_update_kernel(int64_t n, int k, doubl
   block_col_partials<KP>(part, k, s_buf, partials);
 }
 
-// The same for an even k: L lanes per row, two columns per lane as one
-// 16-byte load; per-column sums in the same order as pcg_spmm_dot_kernel.
+// q = A p and per-block, per-column partials of p.q for an even k (operators
+// without a staged copy): L lanes per row, two columns per lane as one
+// 16-byte load.
 template <int L>
 __global__ void __launch_bounds__(kNT) pcg_spmm_dot_vec_kernel(int64_t n, int k, const int32_t* __restrict__ rp,
                                                              const int32_t* __restrict__ ci,
@@ -756,169 +765,7 @@ __global__ void __launch_bounds__(kNT) pcg_spmm_dot_vec_kernel(int64_t n, int k,
     const int c = threadIdx.x;
     double sum = 0.0;
     for (int t = c / 2; t < kNT; t += L) sum += s_buf[2 * t + (c & 1)];
-    partials[(int64_t)blockIdx.x * k + c] = sum;
-  }
-}
-
-// q = A p on the sliced-ELL copy (one lane per row in its layout) for an even
-// k, with per-block, per-column partials of p.q.  As sell_multi_kernel, L
-// lanes per row own two columns each; a unit is one slice quarter (64 / L
-// rows), walked by the block's wavefronts one front per XCD.
-template <int L, int CW>
-__global__ void __launch_bounds__(kNT) pcg_sell_multi_dot_kernel(int64_t n, int k, int64_t nslices, SellView S,
-                                                                const double* __restrict__ sv,
-                                                                const double* __restrict__ p, double* __restrict__ q,
-                                                                double* __restrict__ partials) {
-  typedef double vec __attribute__((ext_vector_type(CW)));
-  constexpr int RW = 64 / L;
-  __shared__ double s_buf[CW * kNT];
-  const int lane = threadIdx.x & 63;
-  const int c0 = (lane % L) * CW;
-  const bool on = c0 < k;
-  const XcdRows R = xcd_rows(nslices * L, kNT / 64);
-  vec part = (vec)(0.0);
-  for (int64_t u = R.first + (threadIdx.x >> 6); u < R.hi; u += R.step) {
-    const int unit = __builtin_amdgcn_readfirstlane((int)u);
-    const int slice = unit / L;
-    const int rl = (unit % L) * RW + lane / L;
-    const int off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
-    const int w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - off) >> 6);
-    const int32_t* wp = S.swin + slice * kSellWindows;
-    const SellWin W{__builtin_amdgcn_readfirstlane(wp[0]), __builtin_amdgcn_readfirstlane(wp[1]),
-                    __builtin_amdgcn_readfirstlane(wp[2]), __builtin_amdgcn_readfirstlane(wp[3]),
-                    __builtin_amdgcn_readfirstlane(wp[4]), __builtin_amdgcn_readfirstlane(wp[5]),
-                    __builtin_amdgcn_readfirstlane(wp[6]), __builtin_amdgcn_readfirstlane(wp[7])};
-    const int64_t pos = (int64_t)slice * 64 + rl;
-    if (!on || pos >= n) continue;
-    const double* vp = sv + off + rl;
-    vec acc = (vec)(0.0);
-    if (W.b0 >= 0) {
-      const uint16_t* cp = S.sc16 + off + rl;
-      int j = 0;
-      for (; j + 4 <= w; j += 4) {
-        const int j0 = sell_col(cp[64 * j], W), j1 = sell_col(cp[64 * (j + 1)], W);
-        const int j2 = sell_col(cp[64 * (j + 2)], W), j3 = sell_col(cp[64 * (j + 3)], W);
-        const double v0 = vp[64 * j], v1 = vp[64 * (j + 1)], v2 = vp[64 * (j + 2)], v3 = vp[64 * (j + 3)];
-        const vec g0 = *(const vec*)(p + (int64_t)j0 * k + c0), g1 = *(const vec*)(p + (int64_t)j1 * k + c0);
-        const vec g2 = *(const vec*)(p + (int64_t)j2 * k + c0), g3 = *(const vec*)(p + (int64_t)j3 * k + c0);
-        acc += v0 * g0;
-        acc += v1 * g1;
-        acc += v2 * g2;
-        acc += v3 * g3;
-      }
-      for (; j < w; ++j) acc += vp[64 * j] * *(const vec*)(p + (int64_t)sell_col(cp[64 * j], W) * k + c0);
-    } else {
-      const int32_t* cp = S.sc + off + rl;
-      for (int j = 0; j < w; ++j) acc += vp[64 * j] * *(const vec*)(p + (int64_t)cp[64 * j] * k + c0);
-    }
-    if (S.sd64) acc += S.sd64[pos] * *(const vec*)(p + pos * k + c0);  // the diagonal term, last
-    *(vec*)(q + pos * k + c0) = acc;
-    part += acc * *(const vec*)(p + pos * k + c0);
-  }
-#pragma unroll
-  for (int j = 0; j < CW; ++j) s_buf[CW * threadIdx.x + j] = part[j];
-  __syncthreads();
-  if ((int)threadIdx.x < k) {
-    const int c = threadIdx.x;
-    double sum = 0.0;
-    for (int t = c / CW; t < kNT; t += L) sum += s_buf[CW * t + (c % CW)];
-    partials[(int64_t)blockIdx.x * k + c] = sum;
-  }
-}
-
-// Last level-0 smoothing step for k columns (a multiple of 4) on the FP32
-// sliced copy, with per-block, per-column partials of r.z (r the FP64 Krylov
-// residual, z the step's FP32 output, which is written; d is not, the step
-// being the last).  Lanes and units as in pcg_sell_multi_dot_kernel (L lanes
-// per row, 4 columns each, one sweep front per XCD); per column z is what
-// sell_multi_kernel computes for the same step.
-template <int MODE, int L>
-__global__ void __launch_bounds__(kNT) sell_multi_out_kernel(int64_t n, int k, int64_t nslices, SellView S,
-                                                           const float* __restrict__ sv, const float* __restrict__ x,
-                                                           const float* __restrict__ b,
-                                                           const float* __restrict__ dinv,
-                                                           const float* __restrict__ d, float* __restrict__ xn,
-                                                           float c1, float c2, const double* __restrict__ r,
-                                                           double* __restrict__ partials) {
-  typedef float vec __attribute__((ext_vector_type(4)));
-  constexpr int RW = 64 / L;
-  __shared__ double s_buf[4 * kNT];
-  const int lane = threadIdx.x & 63;
-  const int c0 = (lane % L) * 4;
-  const bool on = c0 < k;
-  const XcdRows R = xcd_rows(nslices * L, kNT / 64);
-  double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
-  for (int64_t u = R.first + (threadIdx.x >> 6); u < R.hi; u += R.step) {
-    const int unit = __builtin_amdgcn_readfirstlane((int)u);
-    const int slice = unit / L;
-    const int rl = (unit % L) * RW + lane / L;
-    const int off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
-    const int w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - off) >> 6);
-    const int32_t* wp = S.swin + slice * kSellWindows;
-    const SellWin W{__builtin_amdgcn_readfirstlane(wp[0]), __builtin_amdgcn_readfirstlane(wp[1]),
-                    __builtin_amdgcn_readfirstlane(wp[2]), __builtin_amdgcn_readfirstlane(wp[3]),
-                    __builtin_amdgcn_readfirstlane(wp[4]), __builtin_amdgcn_readfirstlane(wp[5]),
-                    __builtin_amdgcn_readfirstlane(wp[6]), __builtin_amdgcn_readfirstlane(wp[7])};
-    const int64_t pos = (int64_t)slice * 64 + rl;
-    if (!on || pos >= n) continue;
-    const float* vp = sv + off + rl;
-    vec acc = (vec)(0.0f);
-    if (W.b0 >= 0) {
-      const uint16_t* cp = S.sc16 + off + rl;
-      int q = 0;
-      for (; q + 4 <= w; q += 4) {
-        const int j0 = sell_col(cp[64 * q], W), j1 = sell_col(cp[64 * (q + 1)], W);
-        const int j2 = sell_col(cp[64 * (q + 2)], W), j3 = sell_col(cp[64 * (q + 3)], W);
-        const float v0 = vp[64 * q], v1 = vp[64 * (q + 1)], v2 = vp[64 * (q + 2)], v3 = vp[64 * (q + 3)];
-        const vec g0 = *(const vec*)(x + (int64_t)j0 * k + c0), g1 = *(const vec*)(x + (int64_t)j1 * k + c0);
-        const vec g2 = *(const vec*)(x + (int64_t)j2 * k + c0), g3 = *(const vec*)(x + (int64_t)j3 * k + c0);
-        acc += v0 * g0;
-        acc += v1 * g1;
-        acc += v2 * g2;
-        acc += v3 * g3;
-      }
-      for (; q < w; ++q) acc += vp[64 * q] * *(const vec*)(x + (int64_t)sell_col(cp[64 * q], W) * k + c0);
-    } else {
-      const int32_t* cp = S.sc + off + rl;
-      int q = 0;
-      for (; q + 4 <= w; q += 4) {
-        const int j0 = cp[64 * q], j1 = cp[64 * (q + 1)], j2 = cp[64 * (q + 2)], j3 = cp[64 * (q + 3)];
-        const float v0 = vp[64 * q], v1 = vp[64 * (q + 1)], v2 = vp[64 * (q + 2)], v3 = vp[64 * (q + 3)];
-        const vec g0 = *(const vec*)(x + (int64_t)j0 * k + c0), g1 = *(const vec*)(x + (int64_t)j1 * k + c0);
-        const vec g2 = *(const vec*)(x + (int64_t)j2 * k + c0), g3 = *(const vec*)(x + (int64_t)j3 * k + c0);
-        acc += v0 * g0;
-        acc += v1 * g1;
-        acc += v2 * g2;
-        acc += v3 * g3;
-      }
-      for (; q < w; ++q) acc += vp[64 * q] * *(const vec*)(x + (int64_t)cp[64 * q] * k + c0);
-    }
-    const int64_t idx = pos * k + c0;
-    if (S.sd32) acc += S.sd32[pos] * *(const vec*)(x + idx);  // the diagonal term, last
-    vec z;
-    if (MODE == kJacobi) {
-      z = *(const vec*)(x + idx) + (c1 * dinv[pos]) * (*(const vec*)(b + idx) - acc);
-    } else {  // kCheb
-      const vec rr = dinv[pos] * (*(const vec*)(b + idx) - acc);
-      const vec dn = (c1 != 0.0f ? c1 * *(const vec*)(d + idx) : (vec)(0.0f)) + c2 * rr;
-      z = *(const vec*)(x + idx) + dn;
-    }
-    *(vec*)(xn + idx) = z;
-    p0 += r[idx] * (double)z[0];
-    p1 += r[idx + 1] * (double)z[1];
-    p2 += r[idx + 2] * (double)z[2];
-    p3 += r[idx + 3] * (double)z[3];
-  }
-  s_buf[4 * threadIdx.x] = p0;
-  s_buf[4 * threadIdx.x + 1] = p1;
-  s_buf[4 * threadIdx.x + 2] = p2;
-  s_buf[4 * threadIdx.x + 3] = p3;
-  __syncthreads();
-  if ((int)threadIdx.x < k) {
-    const int c = threadIdx.x;
-    double sum = 0.0;
-    for (int t = c / 4; t < kNT; t += L) sum += s_buf[4 * t + (c % 4)];
-    partials[(int64_t)blockIdx.x * k + c] = sum;
+    partials[(int64_t)c * gridDim.x + blockIdx.x] = sum;
   }
 }
 
@@ -938,61 +785,57 @@ __global__ void __launch_bounds__(kNT) pcg_dot_kernel(int64_t n, int k, const do
 
 enum FinishMode { F_STORE = 0, F_ALPHA = 1, F_RR = 2, F_BETA = 3, F_FLEX = 4 };
 
-// one block: column totals of nb partials, then the scalar update
+// one block per column: the total of its nb partials, then the scalar update
 // 1024 threads so that ~16k partials take a few rounds of independent loads.
+// (One block walking all columns took 40 us for 16.)
 constexpr int kFinNT = 1024;
 
 __global__ void __launch_bounds__(kFinNT) pcg_finish_kernel(int nb, int k, const double* __restrict__ partials,
                                                           double* __restrict__ scal, int mode, int slot, double tol2,
                                                           double* __restrict__ host_act) {
   __shared__ double s_buf[kFinNT / 64];
-  __shared__ double s_seq;
-  // |r|^2 finishes are numbered on the device; record n goes to host record n % 2
-  if (mode == F_RR && threadIdx.x == 0) {
-    s_seq = scal[S_SEQ * k] + 1.0;
-    scal[S_SEQ * k] = s_seq;
-  }
-  __syncthreads();
-  double* rec = (mode == F_RR && host_act) ? host_act + ((int64_t)s_seq & 1) * kActRec : nullptr;
-  for (int c = 0; c < k; ++c) {
-    double v = 0.0;
+  const int c = blockIdx.x;
+  const double* __restrict__ part = partials + (int64_t)c * nb;
+  double v = 0.0;
 #pragma unroll 8
-    for (int b = threadIdx.x; b < nb; b += kFinNT) v += partials[(int64_t)b * k + c];
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) s_buf[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      v = 0.0;
-      for (int w = 0; w < kFinNT / 64; ++w) v += s_buf[w];
-      if (mode == F_STORE) {
-        scal[slot * k + c] = v;
-      } else if (mode == F_ALPHA) {
-        scal[S_PQ * k + c] = v;
-        scal[S_ALPHA * k + c] = (scal[S_ACT * k + c] != 0.0 && v != 0.0) ? scal[S_RZ * k + c] / v : 0.0;
-      } else if (mode == F_RR) {
-        scal[S_RR * k + c] = v;
-        bool act = scal[S_ACT * k + c] != 0.0 && v > tol2 * scal[S_BB * k + c];
-        scal[S_ACT * k + c] = act ? 1.0 : 0.0;
-        if (rec) {
-          rec[c] = act ? 1.0 : 0.0;
-          rec[64 + c] = v;
-        }
-      } else if (mode == F_FLEX) {
-        // v = z.q with q = A p of the last step: z.r_old = z.r + alpha z.q, so
-        // the flexible (Polak-Ribiere) beta = (z.r - z.r_old) / rz_old =
-        // -alpha z.q / rz_old; z.r was stored in S_RZN
-        const double rz = scal[S_RZ * k + c];
-        scal[S_BETA * k + c] = (scal[S_ACT * k + c] != 0.0 && rz != 0.0) ? -scal[S_ALPHA * k + c] * v / rz : 0.0;
-        scal[S_RZ * k + c] = scal[S_RZN * k + c];
-      } else {
-        double rz = scal[S_RZ * k + c];
-        scal[S_BETA * k + c] = (scal[S_ACT * k + c] != 0.0 && rz != 0.0) ? v / rz : 0.0;
-        scal[S_RZ * k + c] = v;
-      }
+  for (int b = threadIdx.x; b < nb; b += kFinNT) v += part[b];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) s_buf[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  v = 0.0;
+  for (int w = 0; w < kFinNT / 64; ++w) v += s_buf[w];
+  if (mode == F_STORE) {
+    scal[slot * k + c] = v;
+  } else if (mode == F_ALPHA) {
+    scal[S_PQ * k + c] = v;
+    scal[S_ALPHA * k + c] = (scal[S_ACT * k + c] != 0.0 && v != 0.0) ? scal[S_RZ * k + c] / v : 0.0;
+  } else if (mode == F_RR) {
+    // |r|^2 finishes are numbered on the device (every column counts its
+    // own); record n goes to host record n % 2
+    const double seq = scal[S_SEQ * k + c] + 1.0;
+    scal[S_SEQ * k + c] = seq;
+    scal[S_RR * k + c] = v;
+    const bool act = scal[S_ACT * k + c] != 0.0 && v > tol2 * scal[S_BB * k + c];
+    scal[S_ACT * k + c] = act ? 1.0 : 0.0;
+    if (host_act) {
+      double* rec = host_act + ((int64_t)seq & 1) * kActRec;
+      rec[c] = act ? 1.0 : 0.0;
+      rec[64 + c] = v;
+      if (c == 0) rec[128] = seq;  // read by the host after this kernel completed
     }
-    __syncthreads();
+  } else if (mode == F_FLEX) {
+    // v = z.q with q = A p of the last step: z.r_old = z.r + alpha z.q, so
+    // the flexible (Polak-Ribiere) beta = (z.r - z.r_old) / rz_old =
+    // -alpha z.q / rz_old; z.r was stored in S_RZN
+    const double rz = scal[S_RZ * k + c];
+    scal[S_BETA * k + c] = (scal[S_ACT * k + c] != 0.0 && rz != 0.0) ? -scal[S_ALPHA * k + c] * v / rz : 0.0;
+    scal[S_RZ * k + c] = scal[S_RZN * k + c];
+  } else {
+    const double rz = scal[S_RZ * k + c];
+    scal[S_BETA * k + c] = (scal[S_ACT * k + c] != 0.0 && rz != 0.0) ? v / rz : 0.0;
+    scal[S_RZ * k + c] = v;
   }
-  if (rec && threadIdx.x == 0) rec[128] = s_seq;  // read by the host after this kernel completed
 }
 
 // p = z + beta p
@@ -1049,8 +892,8 @@ template <typename T>
 double matrix_bytes(const Csr& A, int k) {
   const bool sell = k == 1 && A.nslices > 0;
   const double nd = sell ? (double)A.nnz_sdiag : 0.0;  // diagonal outside the slices: no column code
-  if (sell && A.lds_bs > 0)  // 16-bit LDS indices, and each block's column list
-    return (double)A.nnz * sizeof(T) + 2.0 * ((double)A.nnz - nd) + 4.0 * (double)A.lcols.size();
+  if (sell && A.lds.bs > 0)  // 16-bit LDS indices, and each block's column list
+    return (double)A.nnz * sizeof(T) + 2.0 * ((double)A.nnz - nd) + 4.0 * (double)A.lds.lcols.size();
   const double nc = sell ? (double)A.nnz_compact : 0.0;
   return (double)A.nnz * sizeof(T) + 2.0 * nc + 4.0 * ((double)A.nnz - nd - nc);
 }
@@ -1082,46 +925,11 @@ bool fused_out(const Level0Io* io, const Csr& A, int k) {
 }
 
 // The last level-0 smoothing step for k > 1 columns with r.z partials
-// (io->r64 and io->partials, no io->z64) on the FP32 sliced copy
+// (io->r64 and io->partials, no io->z64) on the FP32 staged copy
 template <typename T>
 bool multi_out(const Level0Io* io, const Csr& A, int k) {
-  return std::is_same<T, float>::value && io && io->r64 && io->partials && !io->z64 && k > 1 && k % 4 == 0 &&
-         k <= 64 && A.nslices > 0 && A.s32.size() > 0 && A.srow.size() == 0 && A.sell_g == 1;
-}
-
-// launches sell_multi_out_kernel; returns the partial blocks written
-template <int MODE>
-unsigned launch_multi_out(const Csr& A, int k, const float* x, const float* b, const float* dinv, const float* d,
-                          float* xn, float c1, float c2, const double* r, double* partials, hipStream_t s) {
-  const int L = pow2_at_least(k / 4);
-  int64_t g = (A.nslices * L + kNT / 64 - 1) / (kNT / 64);
-  if (g > 4096) g = 4096;
-  const SellView S = sell_view(A);
-  const float* sv = A.s32.get();
-  switch (L) {
-    case 1:
-      sell_multi_out_kernel<MODE, 1><<<(unsigned)g, kNT, 0, s>>>(A.n, k, A.nslices, S, sv, x, b, dinv, d, xn, c1, c2,
-                                                                 r, partials);
-      break;
-    case 2:
-      sell_multi_out_kernel<MODE, 2><<<(unsigned)g, kNT, 0, s>>>(A.n, k, A.nslices, S, sv, x, b, dinv, d, xn, c1, c2,
-                                                                 r, partials);
-      break;
-    case 4:
-      sell_multi_out_kernel<MODE, 4><<<(unsigned)g, kNT, 0, s>>>(A.n, k, A.nslices, S, sv, x, b, dinv, d, xn, c1, c2,
-                                                                 r, partials);
-      break;
-    case 8:
-      sell_multi_out_kernel<MODE, 8><<<(unsigned)g, kNT, 0, s>>>(A.n, k, A.nslices, S, sv, x, b, dinv, d, xn, c1, c2,
-                                                                 r, partials);
-      break;
-    default:
-      sell_multi_out_kernel<MODE, 16><<<(unsigned)g, kNT, 0, s>>>(A.n, k, A.nslices, S, sv, x, b, dinv, d, xn, c1,
-                                                                  c2, r, partials);
-      break;
-  }
-  HIP_LAUNCH_CHECK();
-  return (unsigned)g;
+  return std::is_same<T, float>::value && io && io->r64 && io->partials && !io->z64 && k <= 64 &&
+         multi_staged<float>(A, k) && A.srow.size() == 0;
 }
 
 // nu steps of the smoother from x = 0 (zero == true) or from the given x.
@@ -1161,16 +969,16 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
     HIP_LAUNCH_CHECK();
   };
   auto last_step = [&](int mode, T* cur, double c1, double c2) {
-    if (A.lds_bs > 0) {
-      const size_t lds = sizeof(float) * (size_t)A.lds_maxc;
+    if (A.lds.bs > 0) {
+      const size_t lds = sizeof(float) * (size_t)A.lds.maxc;
       lds_launch(A, 4, [&](auto head, unsigned nb, unsigned nt) {
         if (mode == kJacobi)
           sell_lds_out_kernel<kJacobi, head.value><<<nb, nt, lds, s>>>(
-              A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(), (const float*)cur, (const float*)b,
+              A.n, A.nslices, sell_view(A), lds_view(A.lds), A.s32.get(), (const float*)cur, (const float*)b,
               (const float*)dinv, (const float*)d, (float)c1, (float)c2, io->r64, io->z64, io->partials);
         else
           sell_lds_out_kernel<kCheb, head.value><<<nb, nt, lds, s>>>(
-              A.n, A.nslices, sell_view(A), lds_view(A), A.s32.get(), (const float*)cur, (const float*)b,
+              A.n, A.nslices, sell_view(A), lds_view(A.lds), A.s32.get(), (const float*)cur, (const float*)b,
               (const float*)dinv, (const float*)d, (float)c1, (float)c2, io->r64, io->z64, io->partials);
         io->nb = nb;
       });
@@ -1206,8 +1014,10 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
       }
       if constexpr (std::is_same<T, float>::value) {
         if (outk && step == nu - 1) {
-          io->nb = launch_multi_out<kJacobi>(A, k, cur, b, dinv, nullptr, nxt, (float)S.omega, 0.0f, io->r64,
-                                             io->partials, s);
+          launch_lds_multi<float, kJacobi, 2>(A, k, cur, nullptr, b, dinv, nullptr, nxt, (float)S.omega, 0.0f, io->r64,
+                                              io->partials, s);
+          HIP_LAUNCH_CHECK();
+          io->nb = multi_blocks(A);
           return nxt;
         }
       }
@@ -1243,7 +1053,10 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
     }
     if constexpr (std::is_same<T, float>::value) {
       if (outk && step == nu - 1) {
-        io->nb = launch_multi_out<kCheb>(A, k, cur, b, dinv, d, nxt, (float)c1, (float)c2, io->r64, io->partials, s);
+        launch_lds_multi<float, kCheb, 2>(A, k, cur, nullptr, b, dinv, d, nxt, (float)c1, (float)c2, io->r64,
+                                          io->partials, s);
+        HIP_LAUNCH_CHECK();
+        io->nb = multi_blocks(A);
         return nxt;
       }
     }
@@ -1375,13 +1188,13 @@ unsigned vcycle0_half(Handle& h, const double* r64, double* z64, double* partial
   const int nu_post = h.prm.postInnerIters * (h.prm.postRelaxes > 0 ? h.prm.postRelaxes : 1);
   const unsigned g = grid_for(O.nslices, kNT / 64);
   const SellView V = sell_view(O);
-  // LDS-staged copy when its lists exist: one block per O.lds_bs slices
-  const bool staged = O.lds_bs > 0;
-  const LdsView LV_ = staged ? lds_view(O) : LdsView{};
-  const unsigned gl = staged ? (unsigned)((O.nslices + O.lds_bs - 1) / O.lds_bs) : 0;
-  const size_t ldsb = staged ? sizeof(float) * (size_t)O.lds_maxc : 0;
+  // LDS-staged copy when its lists exist: one block per O.lds.bs slices
+  const bool staged = O.lds.bs > 0;
+  const LdsView LV_ = staged ? lds_view(O.lds) : LdsView{};
+  const unsigned gl = staged ? (unsigned)((O.nslices + O.lds.bs - 1) / O.lds.bs) : 0;
+  const size_t ldsb = staged ? sizeof(float) * (size_t)O.lds.maxc : 0;
   // algorithmic bytes: FP16 value + column code per off-diagonal, and y, b^, diag (+ d r/w), y_new
-  const double mbytes = staged ? 2.0 * (double)O.nnz + 2.0 * (double)O.nnz + 4.0 * (double)O.lcols.size()
+  const double mbytes = staged ? 2.0 * (double)O.nnz + 2.0 * (double)O.nnz + 4.0 * (double)O.lds.lcols.size()
                                : 2.0 * (double)O.nnz + 2.0 * (double)O.nnz_compact +
                                      4.0 * ((double)O.nnz - O.nnz_compact);
   const double step_bytes = mbytes + 4.0 * n * (S.type ? 6.0 : 4.0);
@@ -1738,14 +1551,35 @@ void apply_level_int(Handle& h, int lvl, int which, const double* x, double* y) 
   }
 }
 
+int padded_columns(const Handle&, int k) {
+  // fours: whole 16-byte FP32 groups in every kernel.  5 columns in 8 against a
+  // lane per column with 3 of 8 idle (61 x 58 x 73, FP64 solve 16.4 -> 9.7 ms):
+  // the entry-split and staged kernels need groups, and the kernels that took
+  // any count walked the coarse levels' long rows serially (43 us for 832 rows)
+  if (k <= 1) return 1;
+  return (k + 3) / 4 * 4;
+}
+
 void ensure_krylov(Handle& h, int k) {
   const int64_t n = h.A.n;
+  if (k > 1) {
+    // staging lists of blocks of kMultiSlices slices beside the one-column
+    // lists of larger blocks (whose x rows do not fit LDS two blocks a CU)
+    auto lists = [&](Csr& A) {
+      if (A.nslices > 0 && A.sell_g == 1 && A.lds.bs > kMultiSlices && A.ldm.bs == 0)
+        build_lds(A, kMultiSlices, A.ldm, h.stream);
+    };
+    lists(h.A);
+    for (auto& Lp : h.H.levels) {
+      lists(Lp->A);
+    }
+  }
   if (h.kcap < k) {
     ++h.gen;
     h.kx.resize(n * k); h.kr.resize(n * k); h.kp.resize(n * k); h.kq.resize(n * k);
     h.kz.resize(n * k); h.kb.resize(n * k);
     h.ubuf.resize(n * k); h.ubuf2.resize(n * k);
-    h.partials.resize((size_t)std::max<int64_t>(4096, n / 256 + 2) * 64);
+    h.partials.resize((size_t)std::max<int64_t>(4096, n / 128 + 2) * 64);
     h.scal.resize((size_t)S_COUNT * 64);
     if (!h.h_scal) HIP_CHECK(hipHostMalloc((void**)&h.h_scal, sizeof(double) * S_COUNT * 64, hipHostMallocDefault));
     if (!h.h_act) {
@@ -1813,7 +1647,7 @@ void run_iteration(Handle& h, int k, double tol2, Fn&& body) {
 }
 
 void finish(Handle& h, int nb, int k, int mode, int slot, double tol2 = 0.0) {
-  pcg_finish_kernel<<<1, kFinNT, 0, h.stream>>>(nb, k, h.partials.get(), h.scal.get(), mode, slot, tol2,
+  pcg_finish_kernel<<<(unsigned)k, kFinNT, 0, h.stream>>>(nb, k, h.partials.get(), h.scal.get(), mode, slot, tol2,
                                                  mode == F_RR ? h.d_act : nullptr);
   HIP_LAUNCH_CHECK();
 }
@@ -1872,11 +1706,11 @@ void launch_sell_dot(Handle& h) {
   const Csr& A = h.A;
   if (A.srow.size() || A.sell_g != 1)
     fail(FEM_ERR_STATE, "the operator's sliced-ELL copy must keep the row order with one lane per row");
-  if (A.lds_bs > 0) {
+  if (A.lds.bs > 0) {
     unsigned blocks = 0;
     lds_launch(A, 8, [&](auto head, unsigned nb, unsigned nt) {
-      pcg_sell_lds_dot_kernel<head.value><<<nb, nt, sizeof(double) * (size_t)A.lds_maxc, h.stream>>>(
-          A.n, A.nslices, sell_view(A), lds_view(A), A.s64.get(), h.kp.get(), h.kq.get(), h.partials.get());
+      pcg_sell_lds_dot_kernel<head.value><<<nb, nt, sizeof(double) * (size_t)A.lds.maxc, h.stream>>>(
+          A.n, A.nslices, sell_view(A), lds_view(A.lds), A.s64.get(), h.kp.get(), h.kq.get(), h.partials.get());
       blocks = nb;
     });
     HIP_LAUNCH_CHECK();
@@ -1901,29 +1735,13 @@ void launch_spmv_dot(Handle& h) {
   finish(h, (int)g, 1, F_ALPHA, 0);
 }
 
-// FP64 columns per lane of the multi-column sliced operator + dot (as sell_multi_cols)
-constexpr int kDotCols = 4;
-
-template <int KP>
+template <int L>
 void launch_spmm_dot(Handle& h, int k) {
   const Csr& A = h.A;
-  int64_t g = (A.n * KP + kNT - 1) / kNT;
+  int64_t g = (A.n * L + kNT - 1) / kNT;
   if (g > 4096) g = 4096;
-  if (k % kDotCols == 0 && A.nslices > 0 && A.sell_g == 1 && A.s64.size() && A.srow.size() == 0) {
-    constexpr int L = KP >= kDotCols ? KP / kDotCols : 1;
-    int64_t gs = (A.nslices * L + kNT / 64 - 1) / (kNT / 64);
-    if (gs > 4096) gs = 4096;
-    g = gs;
-    pcg_sell_multi_dot_kernel<L, kDotCols><<<(unsigned)g, kNT, 0, h.stream>>>(
-        A.n, k, A.nslices, sell_view(A), A.s64.get(), h.kp.get(), h.kq.get(), h.partials.get());
-  } else if (k % 2 == 0) {
-    // KP >= k, so KP / 2 lanes per row cover the k / 2 column pairs
-    pcg_spmm_dot_vec_kernel<(KP >= 2 ? KP / 2 : 1)><<<(unsigned)g, kNT, 0, h.stream>>>(
-        A.n, k, A.rp.get(), A.ci.get(), A.v64.get(), h.kp.get(), h.kq.get(), h.partials.get());
-  } else {
-    pcg_spmm_dot_kernel<KP><<<(unsigned)g, kNT, 0, h.stream>>>(A.n, k, A.rp.get(), A.ci.get(), A.v64.get(),
-                                                               h.kp.get(), h.kq.get(), h.partials.get());
-  }
+  pcg_spmm_dot_vec_kernel<L><<<(unsigned)g, kNT, 0, h.stream>>>(A.n, k, A.rp.get(), A.ci.get(), A.v64.get(), h.kp.get(),
+                                                                h.kq.get(), h.partials.get());
   HIP_LAUNCH_CHECK();
   finish(h, (int)g, k, F_ALPHA, 0);
 }
@@ -1941,14 +1759,19 @@ void spmv_dot(Handle& h, int k) {
       case 32: launch_spmv_dot<32>(h); break;
       default: launch_spmv_dot<64>(h); break;
     }
+  } else if (multi_staged<double>(A, k) && A.srow.size() == 0) {
+    launch_lds_multi<double, kAssign, 1>(A, k, h.kp.get(), h.kq.get(), nullptr, (const double*)nullptr, nullptr,
+                                         nullptr, 0.0, 0.0, nullptr, h.partials.get(), h.stream);
+    HIP_LAUNCH_CHECK();
+    finish(h, (int)multi_blocks(A), k, F_ALPHA, 0);
   } else {
-    switch (pow2_at_least(k)) {
+    switch (pow2_at_least(k / 2)) {
+      case 1: launch_spmm_dot<1>(h, k); break;
       case 2: launch_spmm_dot<2>(h, k); break;
       case 4: launch_spmm_dot<4>(h, k); break;
       case 8: launch_spmm_dot<8>(h, k); break;
       case 16: launch_spmm_dot<16>(h, k); break;
-      case 32: launch_spmm_dot<32>(h, k); break;
-      default: launch_spmm_dot<64>(h, k); break;
+      default: launch_spmm_dot<32>(h, k); break;
     }
   }
 }
@@ -2231,9 +2054,9 @@ void apply_preconditioner_noalloc(Handle& h, const double* r_user, double* z_use
   double* r = base;
   double* z = base + kNoAllocRows;
   double* partials = base + 2 * kNoAllocRows;
-  gather_user_to_int(h, r_user, r, 1);
+  gather_user_to_int(h, r_user, r, 1, 1);
   precondition(h, r, z, 1, partials);
-  scatter_int_to_user(h, z, z_user, 1);
+  scatter_int_to_user(h, z, z_user, 1, 1);
 }
 
 }  // namespace fem

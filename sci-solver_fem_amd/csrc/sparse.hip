@@ -1239,11 +1239,8 @@ void build_sell(Csr& A, bool with_f32, hipStream_t s, int64_t sort_window, bool 
   A.sd64.release();
   A.sd32.release();
   A.nnz_sdiag = 0;
-  A.lds_bs = 0;
-  A.lds_maxc = 0;
-  A.lc.release();
-  A.lcs.release();
-  A.lcols.release();
+  A.lds.clear();
+  A.ldm.clear();
   if (split_diag) {
     if (A.n != A.m || lanes != 1 || sort_window > 0 || with_f16)
       fail(FEM_ERR_ARG, "sliced ELL: the diagonal is split off square matrices in row order only");
@@ -1354,12 +1351,8 @@ void build_sell(Csr& A, bool with_f32, hipStream_t s, int64_t sort_window, bool 
   HIP_CHECK(hipStreamSynchronize(s));
 }
 
-void build_lds(Csr& A, int bs, hipStream_t s) {
-  A.lds_bs = 0;
-  A.lds_maxc = 0;
-  A.lc.release();
-  A.lcs.release();
-  A.lcols.release();
+void build_lds(const Csr& A, int bs, LdsList& out, hipStream_t s) {
+  out.clear();
   if (A.nslices <= 0 || A.sell_g != 1 || bs <= 0) return;
   if (bs > kLdsMaxSlices) fail(FEM_ERR_ARG, "LDS staging: at most 8 slices per block");
   const int64_t ns = A.nslices;
@@ -1406,11 +1399,11 @@ void build_lds(Csr& A, int bs, hipStream_t s) {
     HIP_LAUNCH_CHECK();
   }
   HIP_CHECK(hipStreamSynchronize(s));
-  A.lc = std::move(lc);
-  A.lcs = std::move(lcs);
-  A.lcols = std::move(lcols);
-  A.lds_maxc = maxc;
-  A.lds_bs = bs;
+  out.lc = std::move(lc);
+  out.lcs = std::move(lcs);
+  out.lcols = std::move(lcols);
+  out.maxc = maxc;
+  out.bs = bs;
 }
 
 void csr_transpose(const Csr& P, Csr& R, hipStream_t s) {
