@@ -166,6 +166,10 @@ int fem_read_matlab_sparse(fem_handle* h, const char* filename);
 /* Replace the per-element conductivity (user element order) and reassemble
  * in place on the device; the hierarchy is rebuilt by the next setup/solve. */
 int fem_update_kappa(fem_handle* h, const double* kappa);
+/* The same with kappa in device memory (ne doubles, on the handle's device):
+ * no copy through the host.  The caller's writes to kappa must be ordered
+ * before the handle's stream. */
+int fem_update_kappa_device(fem_handle* h, const double* kappa);
 
 /* ---- setup and solve -------------------------------------------------------*/
 /* AMG::setup, src/core/cuda/amg.cu:79-144: aggregation, smoothed prolongator,

@@ -93,6 +93,7 @@ SIGNATURES = {
     "fem_get_matrix_csr": (C.c_int, [_P, _P, _P, _P]),
     "fem_read_matlab_sparse": (C.c_int, [_P, C.c_char_p]),
     "fem_update_kappa": (C.c_int, [_P, _P]),
+    "fem_update_kappa_device": (C.c_int, [_P, _P]),
     "fem_setup": (C.c_int, [_P]),
     "fem_solve": (C.c_int, [_P, _P, _P, C.c_int, C.c_int, C.POINTER(FemSolveInfo)]),
     "fem_adjoint_grad": (C.c_int, [_P, _P, _P, _P, _P, C.c_int, C.POINTER(FemSolveInfo)]),

@@ -431,6 +431,23 @@ int fem_read_matlab_sparse(fem_handle* hh, const char* filename) {
   });
 }
 
+}  // extern "C"
+
+namespace {
+// reassembly for the coefficients at kd (device, user element order), which
+// are checked before any of the handle's data changes
+void reassemble_kappa(Handle& h, const double* kd) {
+  if (check_mesh_device(0, nullptr, 0, h.ne, kd, 0, nullptr, h.stream) & 2)
+    fail(FEM_ERR_NUMERIC, "NaN in element coefficient");
+  set_kappa_user(h, kd);
+  assemble_values(h);
+  HIP_CHECK(hipStreamSynchronize(h.stream));
+  h.H.built = false;
+}
+}  // namespace
+
+extern "C" {
+
 int fem_update_kappa(fem_handle* hh, const double* kappa) {
   if (!hh || !kappa) return FEM_ERR_ARG;
   return guarded(hh, [&]() {
@@ -439,12 +456,17 @@ int fem_update_kappa(fem_handle* hh, const double* kappa) {
     DevBuf<double> ku(h.ne);
     const HostPiece pc = {ku.get(), kappa, sizeof(double) * (size_t)h.ne};
     upload_pieces(&pc, 1, h.stream);
-    if (check_mesh_device(0, nullptr, 0, h.ne, ku.get(), 0, nullptr, h.stream) & 2)
-      fail(FEM_ERR_NUMERIC, "NaN in element coefficient");
-    set_kappa_user(h, ku.get());
-    assemble_values(h);
-    HIP_CHECK(hipStreamSynchronize(h.stream));
-    h.H.built = false;
+    reassemble_kappa(h, ku.get());
+    return (int)FEM_OK;
+  });
+}
+
+int fem_update_kappa_device(fem_handle* hh, const double* kappa) {
+  if (!hh || !kappa) return FEM_ERR_ARG;
+  return guarded(hh, [&]() {
+    Handle& h = *H(hh);
+    if (!h.has_mesh || h.matrix_from_file) fail(FEM_ERR_STATE, "operator is not assembled from a mesh");
+    reassemble_kappa(h, kappa);
     return (int)FEM_OK;
   });
 }
