@@ -420,7 +420,8 @@ class FEMSolver:
 
 def release_cached_memory() -> None:
     """Free the library's reserve of device blocks (temporaries of mesh builds
-    and setups kept for reuse, at most 8 GiB per device)."""
+    and setups and the buffers of closed solvers, kept for reuse, at most 16 GiB
+    per device)."""
     lib().fem_release_cached_memory()
 
 

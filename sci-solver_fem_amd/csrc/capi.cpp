@@ -85,7 +85,7 @@ void create_common(Handle& h, int dim, int64_t nv, const double* xyz, int64_t ne
   h.flags = flags;
   init_device(h);
   {
-    DevPoolScope pool;  // the mesh build's temporaries reuse each other's blocks
+    DevPoolScope pool(h.stream);  // the mesh build's temporaries reuse each other's blocks
     build_mesh_device(h, xyz, conn, kappa);  // validates indices and NaNs on the device
     HIP_CHECK(hipStreamSynchronize(h.stream));
   }
@@ -171,9 +171,15 @@ bool params_shape_changed(const fem_params& a, const fem_params& b) {
 void ensure_setup(Handle& h) {
   if (h.A.n == 0) fail(FEM_ERR_EMPTY, "Error no matrix specified");
   if (!h.H.built) {
-    DevPoolScope pool;  // the setup's temporaries reuse each other's blocks
+    DevPoolScope pool(h.stream);  // the setup's temporaries reuse each other's blocks
     build_hierarchy(h);
   }
+}
+
+// work vectors for k (padded) columns, allocated like the setup's buffers
+void ensure_work(Handle& h, int k) {
+  DevPoolScope pool(h.stream);
+  ensure_krylov(h, k);
 }
 
 // stage nv x k user-order data into internal order on the device (rows of kk
@@ -293,7 +299,9 @@ void fem_release_cached_memory(void) { pool_flush_reserve(); }
 void fem_destroy(fem_handle* hh) {
   Handle* h = H(hh);
   if (!h) return;
-  if (h->stream) (void)hipStreamSynchronize(h->stream);
+  // with the handle's stream drained its buffers are idle and can be reused
+  const bool idle = h->stream && hipStreamSynchronize(h->stream) == hipSuccess;
+  DevRetireScope retire(idle ? h->device : -1);
   if (h->h_scal) (void)hipHostFree(h->h_scal);
   if (h->h_act) (void)hipHostFree(h->h_act);
   if (h->iter_graph) (void)hipGraphExecDestroy(h->iter_graph);
@@ -476,7 +484,7 @@ int fem_setup(fem_handle* hh) {
   return guarded(hh, [&]() {
     Handle& h = *H(hh);
     ensure_setup(h);
-    ensure_krylov(h, 1);  // one-column work vectors (what fem_apply_preconditioner_noalloc needs)
+    ensure_work(h, 1);  // one-column work vectors (what fem_apply_preconditioner_noalloc needs)
     noalloc_init(h);
     return (int)FEM_OK;
   });
@@ -494,7 +502,7 @@ int fem_solve(fem_handle* hh, const double* b, double* x, int nrhs, int on_devic
       setup_ms = h.H.setup_ms;
     }
     const int kk = padded_columns(h, nrhs);
-    ensure_krylov(h, kk);
+    ensure_work(h, kk);
     to_internal(h, b, on_device, h.kb.get(), nrhs, kk);
     to_internal(h, x, on_device, h.kx.get(), nrhs, kk);
     int st = pcg_solve(h, kk, info);
@@ -517,7 +525,7 @@ int fem_adjoint_grad(fem_handle* hh, const double* u, const double* dLdu, double
       ensure_setup(h);
       setup_ms = h.H.setup_ms;
     }
-    ensure_krylov(h, 1);
+    ensure_work(h, 1);
     // K lambda = dL/du (K symmetric), zero initial guess
     to_internal(h, dLdu, on_device, h.kb.get(), 1, 1);
     HIP_CHECK(hipMemsetAsync(h.kx.get(), 0, sizeof(double) * h.A.n, h.stream));
@@ -546,7 +554,7 @@ int fem_element_grad(fem_handle* hh, const double* a, const double* u, double* d
   return guarded(hh, [&]() {
     Handle& h = *H(hh);
     if (!h.has_mesh) fail(FEM_ERR_STATE, "no mesh");
-    ensure_krylov(h, 1);
+    ensure_work(h, 1);
     to_internal(h, a, on_device, h.kq.get(), 1, 1);
     to_internal(h, u, on_device, h.kz.get(), 1, 1);
     double* g = dLdkappa;
@@ -568,7 +576,7 @@ int fem_apply_operator(fem_handle* hh, const double* x, double* y, int nrhs, int
     Handle& h = *H(hh);
     if (h.A.n == 0) fail(FEM_ERR_EMPTY, "Error no matrix specified");
     const int kk = padded_columns(h, nrhs);
-    ensure_krylov(h, kk);
+    ensure_work(h, kk);
     to_internal(h, x, on_device, h.kp.get(), nrhs, kk);
     apply_operator_int(h, h.kp.get(), h.kq.get(), kk);
     from_internal(h, h.kq.get(), y, on_device, nrhs, kk);
@@ -581,7 +589,7 @@ int fem_apply_preconditioner(fem_handle* hh, const double* r, double* z, int on_
   return guarded(hh, [&]() {
     Handle& h = *H(hh);
     ensure_setup(h);
-    ensure_krylov(h, 1);
+    ensure_work(h, 1);
     to_internal(h, r, on_device, h.kr.get(), 1, 1);
     apply_vcycle_fp64(h, h.kr.get(), h.kz.get());
     from_internal(h, h.kz.get(), z, on_device, 1, 1);

@@ -36,14 +36,18 @@ inline void hip_check(hipError_t e, const char* what, const char* file, int line
 // come from the scope's size classes and go back to them when released, so a
 // phase with hundreds of temporaries (the AMG setup) neither waits for the
 // device at every hipFree nor calls hipMalloc for every temporary.  All work
-// of such a phase runs on one stream, which orders a block's reuse after its
-// earlier uses.  When the scope ends its free blocks go, after a device
-// synchronization, to a per-device reserve of at most 8 GiB that later scopes
-// draw from (hipFree of each cost 0.25-0.65 ms, and large frees slow the
-// allocations after them); the reserve is freed by pool_flush_reserve
-// (fem_release_cached_memory) and whenever an allocation fails.
-// Blocks still held when the scope ends (buffers the phase keeps) are freed
-// by hipFree whenever their owner releases them.
+// of such a phase runs on one stream, the handle's, which orders a block's
+// reuse after its earlier uses; blocks that the handle kept from an earlier
+// scope and releases in this one (the hierarchy that a setup replaces) are
+// reused alike.  When the scope ends its free blocks go, once the
+// stream has drained, to a per-device reserve of at most 16 GiB that later scopes
+// draw from (hipFree of each cost 0.1-0.65 ms, and large frees slow the
+// allocations after them: a setup replacing a hierarchy of 1 M rows spent 10
+// of 30 ms in 117 hipFree and 3 in hipMalloc); the reserve is freed by
+// pool_flush_reserve (fem_release_cached_memory) and whenever an allocation
+// fails.  Blocks still held when the scope ends (buffers the phase keeps) go
+// back to the reserve when their handle is destroyed (DevRetireScope), and by
+// hipFree when their owner releases them at any other time.
 void* pool_alloc(size_t bytes);   // null when no scope is active on this thread
 bool pool_release(void* p);       // false when p is not a free-able pool block
 void pool_flush_reserve();
@@ -51,13 +55,27 @@ void* dev_malloc(size_t bytes);   // hipMalloc; on failure the reserve is freed 
 
 class DevPoolScope {
  public:
-  DevPoolScope();
+  explicit DevPoolScope(hipStream_t stream);  // the stream of all the scope's work
   ~DevPoolScope();
   DevPoolScope(const DevPoolScope&) = delete;
   DevPoolScope& operator=(const DevPoolScope&) = delete;
 
  private:
   void* prev_;
+  hipStream_t stream_;
+};
+
+// While alive on a thread, pool blocks of `device` released there go to the
+// reserve.  The caller has synchronized every stream whose work uses them.
+class DevRetireScope {
+ public:
+  explicit DevRetireScope(int device);
+  ~DevRetireScope();
+  DevRetireScope(const DevRetireScope&) = delete;
+  DevRetireScope& operator=(const DevRetireScope&) = delete;
+
+ private:
+  int prev_;
 };
 
 // Host -> device copy of pageable host memory in pieces (destination, source,

@@ -15,12 +15,13 @@ namespace fem {
 namespace {
 
 struct Pool {
-  std::unordered_map<void*, size_t> owned;  // blocks this pool allocated -> size class
+  std::unordered_map<void*, size_t> owned;  // blocks this pool may hand on -> size class
   std::multimap<size_t, void*> free_;       // released blocks by size class
   int device = 0;
 };
 
 thread_local Pool* g_pool = nullptr;
+thread_local int g_retire = -1;  // device whose idle blocks this thread's releases go to the reserve of
 
 // size classes: 256 B, then 2^k (1 + j / 8): at most 12.5 % above the request
 size_t size_class(size_t bytes) {
@@ -31,21 +32,50 @@ size_t size_class(size_t bytes) {
   return (bytes + step - 1) / step * step;
 }
 
-// free blocks of ended scopes, per device, by size class
-constexpr size_t kReserveCap = (size_t)8 << 30;
+// free blocks of ended scopes and destroyed handles, per device, by size
+// class; and every live block that came from a pool, so that it can return
+// to one (process-lifetime objects: handles may be destroyed at exit)
+constexpr size_t kReserveCap = (size_t)16 << 30;  // a 161^3 handle and its temporaries: about 12 GiB
 struct Reserve {
   std::multimap<size_t, void*> blocks;
   size_t bytes = 0;
 };
+struct Block {
+  size_t cls;
+  int device;
+};
 std::mutex g_res_mu;
-std::unordered_map<int, Reserve> g_res;
+std::unordered_map<int, Reserve>& reserves() {
+  static auto* r = new std::unordered_map<int, Reserve>();
+  return *r;
+}
+std::unordered_map<void*, Block>& blocks() {
+  static auto* b = new std::unordered_map<void*, Block>();
+  return *b;
+}
+
+// an idle block into its device's reserve, or freed when that is full (the
+// caller holds g_res_mu)
+void retire_locked(void* p, size_t cls, int device) {
+  Reserve& r = reserves()[device];
+  if (r.bytes + cls <= kReserveCap) {
+    r.blocks.emplace(cls, p);
+    r.bytes += cls;
+  } else {
+    blocks().erase(p);
+    (void)hipFree(p);
+  }
+}
 
 }  // namespace
 
 void pool_flush_reserve() {
   std::lock_guard<std::mutex> lk(g_res_mu);
-  for (auto& dr : g_res) {
-    for (auto& kv : dr.second.blocks) (void)hipFree(kv.second);
+  for (auto& dr : reserves()) {
+    for (auto& kv : dr.second.blocks) {
+      blocks().erase(kv.second);
+      (void)hipFree(kv.second);
+    }
     dr.second.blocks.clear();
     dr.second.bytes = 0;
   }
@@ -74,8 +104,8 @@ void* pool_alloc(size_t bytes) {
   void* p = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_res_mu);
-    auto rt = g_res.find(pl->device);
-    if (rt != g_res.end()) {
+    auto rt = reserves().find(pl->device);
+    if (rt != reserves().end()) {
       auto jt = rt->second.blocks.find(c);
       if (jt != rt->second.blocks.end()) {
         p = jt->second;
@@ -84,21 +114,44 @@ void* pool_alloc(size_t bytes) {
       }
     }
   }
-  if (!p) p = dev_malloc(c);
+  if (!p) {
+    p = dev_malloc(c);
+    std::lock_guard<std::mutex> lk(g_res_mu);
+    blocks()[p] = Block{c, pl->device};
+  }
   pl->owned.emplace(p, c);
   return p;
 }
 
 bool pool_release(void* p) {
   Pool* pl = g_pool;
-  if (!pl) return false;
-  auto it = pl->owned.find(p);
-  if (it == pl->owned.end()) return false;
-  pl->free_.emplace(it->second, p);
-  return true;
+  if (pl) {
+    auto it = pl->owned.find(p);
+    if (it != pl->owned.end()) {
+      pl->free_.emplace(it->second, p);
+      return true;
+    }
+  }
+  std::lock_guard<std::mutex> lk(g_res_mu);
+  auto bt = blocks().find(p);
+  if (bt == blocks().end()) return false;
+  const Block b = bt->second;
+  if (pl && b.device == pl->device) {
+    // a block of an earlier scope (the hierarchy that a setup replaces): its
+    // uses are on this scope's stream, before whatever the block serves next
+    pl->owned.emplace(p, b.cls);
+    pl->free_.emplace(b.cls, p);
+    return true;
+  }
+  if (g_retire == b.device) {
+    retire_locked(p, b.cls, b.device);
+    return true;
+  }
+  blocks().erase(bt);
+  return false;
 }
 
-DevPoolScope::DevPoolScope() : prev_(g_pool) {
+DevPoolScope::DevPoolScope(hipStream_t stream) : prev_(g_pool), stream_(stream) {
   Pool* pl = new Pool();
   (void)hipGetDevice(&pl->device);
   g_pool = pl;
@@ -107,15 +160,16 @@ DevPoolScope::DevPoolScope() : prev_(g_pool) {
 DevPoolScope::~DevPoolScope() {
   Pool* pl = g_pool;
   if (!pl->free_.empty()) {
-    // queued work may still use the blocks: only an idle device hands them on
-    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    // queued work may still use the blocks: they are handed on once the
+    // scope's stream has drained (a device synchronization would also end
+    // another thread's stream capture)
+    const bool idle = hipStreamSynchronize(stream_) == hipSuccess;
     std::lock_guard<std::mutex> lk(g_res_mu);
-    Reserve& r = g_res[pl->device];
     for (auto& kv : pl->free_) {
-      if (idle && r.bytes + kv.first <= kReserveCap) {
-        r.blocks.emplace(kv.first, kv.second);
-        r.bytes += kv.first;
+      if (idle) {
+        retire_locked(kv.second, kv.first, pl->device);
       } else {
+        blocks().erase(kv.second);
         (void)hipFree(kv.second);
       }
     }
@@ -123,6 +177,9 @@ DevPoolScope::~DevPoolScope() {
   delete pl;
   g_pool = static_cast<Pool*>(prev_);
 }
+
+DevRetireScope::DevRetireScope(int device) : prev_(g_retire) { g_retire = device; }
+DevRetireScope::~DevRetireScope() { g_retire = prev_; }
 
 namespace {
 
