@@ -413,52 +413,44 @@ __global__ void hash_vector_kernel(int64_t n, unsigned long long seed, double* _
   v[i] = 0.5 + (double)(z >> 11) * (1.0 / 9007199254740992.0);
 }
 
-// one block: nrm = sqrt(sum of the nb partials, summed in index order)
-__global__ void norm_finish_kernel(int nb, const double* __restrict__ part, double* __restrict__ nrm) {
-  if (threadIdx.x != 0) return;
-  double t = 0.0;
-  // in index order; the loads of a chunk are issued together
-  int b = 0;
-  for (; b + 16 <= nb; b += 16) {
-    double c[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) c[j] = part[b + j];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) t += c[j];
+// v *= 1 / nrm with nrm = sqrt(sum of the nb = kNT partials) when nrm > 0 (a
+// zero or NaN norm leaves v as it is).  Every block adds the partials itself
+// (2 KB, one per thread, the same tree everywhere), block 0 keeps the norm:
+// a launch of one thread walking them took 5 to 7 us per step.
+__global__ void __launch_bounds__(kNT) scale_by_norm_kernel(int64_t n, const double* __restrict__ part,
+                                                          double* __restrict__ nrm, double* __restrict__ v) {
+  __shared__ double s_buf[kNT];
+  __shared__ double s_nrm;
+  const double t = block_sum(part[threadIdx.x], s_buf);
+  if (threadIdx.x == 0) {
+    s_nrm = sqrt(t);
+    if (blockIdx.x == 0) nrm[0] = s_nrm;
   }
-  for (; b < nb; ++b) t += part[b];
-  nrm[0] = sqrt(t);
-}
-
-// v *= 1 / nrm when nrm > 0 (a zero or NaN norm leaves v as it is)
-__global__ void scale_by_norm_kernel(int64_t n, const double* __restrict__ nrm, double* __restrict__ v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const double a = nrm[0];
-  if (i < n && a > 0) v[i] *= 1.0 / a;
+  __syncthreads();
+  const double a = s_nrm;
+  if (!(a > 0)) return;
+  for (int64_t i = (int64_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kNT) v[i] *= 1.0 / a;
 }
 
 // Spectral radius of D^-1 A by power iteration (upper part of the spectrum),
 // on the device with one read-back at the end.
 double estimate_rho(const Csr& A, const double* dinv, hipStream_t s, int iters = 15) {
   const int64_t n = A.n;
-  const int nb = 256;
+  const int nb = kNT;
   DevBuf<double> v(n), w(n), part(nb), nrm(iters + 1);
   hash_vector_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, 12345ull, v.get());
   HIP_LAUNCH_CHECK();
-  auto norm_into = [&](double* x, const double* scale, double* out) {
+  // x (scaled by `scale` first) over its norm, which goes to out
+  auto normalise = [&](double* x, const double* scale, double* out) {
     sumsq_kernel<<<nb, kNT, 0, s>>>(n, x, scale, part.get());
     HIP_LAUNCH_CHECK();
-    norm_finish_kernel<<<1, 64, 0, s>>>(nb, part.get(), out);
+    scale_by_norm_kernel<<<std::min<unsigned>(grid_for(n, kNT), 2048u), kNT, 0, s>>>(n, part.get(), out, x);
     HIP_LAUNCH_CHECK();
   };
-  norm_into(v.get(), nullptr, nrm.get());
-  scale_by_norm_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, nrm.get(), v.get());
-  HIP_LAUNCH_CHECK();
+  normalise(v.get(), nullptr, nrm.get());
   for (int it = 0; it < iters; ++it) {
     spmv64(A, v.get(), w.get(), s);
-    norm_into(w.get(), dinv, nrm.get() + 1 + it);  // w = D^-1 A v and its norm
-    scale_by_norm_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, nrm.get() + 1 + it, w.get());
-    HIP_LAUNCH_CHECK();
+    normalise(w.get(), dinv, nrm.get() + 1 + it);  // w = D^-1 A v over its norm
     std::swap(v, w);
   }
   std::vector<double> h = nrm.to_host(s);
