@@ -1086,6 +1086,274 @@ bool restrict_first(Handle& h, int l, const Csr& R, const T* r, int k) {
   return true;
 }
 
+// Chebyshev coefficients of step `step` of a smoother on [lmin, lmax]
+struct ChebSeq {
+  double theta, delta, sigma, rho_old;
+  explicit ChebSeq(const Smoother& S)
+      : theta(0.5 * (S.lmax + S.lmin)), delta(0.5 * (S.lmax - S.lmin)), sigma(theta / delta), rho_old(delta / theta) {}
+  void next(int step, double& c1, double& c2) {
+    if (step == 0) {
+      c1 = 0.0;
+      c2 = 1.0 / theta;
+    } else {
+      const double rho_new = 1.0 / (2.0 * sigma - rho_old);
+      c1 = rho_new * rho_old;
+      c2 = 2.0 * rho_new / delta;
+      rho_old = rho_new;
+    }
+  }
+};
+
+// ---- the V-cycle's small levels in one launch --------------------------------------
+// One block restricts the residual of the level above, runs the V-cycle of
+// the levels below it and solves the coarsest level, with the levels'
+// matrices and vectors in LDS.  Level by level these are some ten launches,
+// each a few microseconds of launch and load latency for a few thousand
+// entries: 65^2 (297 and 21 rows, FP64) 33 us in ten launches, 20 us here;
+// 1003 x 701 (300 and 19 rows below five levels, FP32) 50 -> 27 us; 97^3
+// (restriction and the 59-row solve only) 16 -> 9.5 us.  A phase is a chain of
+// LDS reads per row, about 1.5 us: with the matrices left in L2 it took 2 us,
+// and with 512 or 256 threads the launch takes 24 and 33 us at 65^2.
+constexpr int kTailLevels = 6;
+constexpr int kTailSteps = 8;
+constexpr int kTailNT = 1024;
+constexpr size_t kTailLds = 150 * 1024;
+// What stays in memory is streamed by one CU, so it has to be little: entries
+// of the restriction into the first level, rows of the coarsest level (its
+// inverse; 13^3, 100 rows: the launch takes 12 us against 5 for the two that
+// use the whole chip)
+constexpr int64_t kTailRnnz = 16384;
+constexpr int64_t kTailCoarse = 64;
+// rows of a smoothed level: 475 rows break even (300 x 280: 4.94 -> 4.89 ms a
+// solve), 689 lose (379 x 321: 4.97 -> 5.19 ms), 271 gain (71 x 55: 2.07 -> 1.80)
+constexpr int64_t kTailRows = 480;
+
+template <typename T>
+struct TailCsr {
+  const int32_t* rp;
+  const int32_t* ci;
+  const T* v;
+  int n, nnz, lg;       // rows, entries, log2 of the lanes per row
+  int o_v, o_rp, o_ci;  // byte offsets of its copy in LDS
+};
+
+template <typename T>
+struct TailLevel {
+  TailCsr<T> A, P, R;
+  const T* dinv;
+  int o_dinv, o_vec;  // LDS: D^-1; x, t, b, d, r
+  T c0;               // first step from zero
+  T pre1[kTailSteps], pre2[kTailSteps], post1[kTailSteps], post2[kTailSteps];
+};
+
+template <typename T>
+struct TailArgs {
+  int nlev;  // smoothed levels, then the coarsest
+  int type, npre, npost;
+  TailCsr<T> R;        // restriction into the first level (in memory)
+  const T* r;          // residual above it
+  T* x;                // its result
+  const double* cinv;  // the coarsest level's inverse
+  int nc, o_coarse;    // LDS: its x and b
+  TailLevel<T> lev[kTailLevels];
+};
+
+// f(row, (M x)_row) for every row, xs(j) = x_j; the block's threads in groups
+// of 2^lg lanes per row
+template <typename T, typename RP, typename CI, typename X, typename F>
+__device__ __forceinline__ void tail_rows(int n, int lg, const RP* rp, const CI* ci, const T* v, X xs, F f) {
+  const int g = 1 << lg, lane = threadIdx.x & (g - 1);
+  for (int row = threadIdx.x >> lg; row < n; row += kTailNT >> lg) {
+    const int e = rp[row + 1];
+    int q = rp[row] + lane;
+    T acc = T(0);
+    for (; q + 3 * g < e; q += 4 * g) {
+      const int j0 = ci[q], j1 = ci[q + g], j2 = ci[q + 2 * g], j3 = ci[q + 3 * g];
+      const T v0 = v[q], v1 = v[q + g], v2 = v[q + 2 * g], v3 = v[q + 3 * g];
+      const T x0 = xs(j0), x1 = xs(j1), x2 = xs(j2), x3 = xs(j3);
+      acc += v0 * x0;
+      acc += v1 * x1;
+      acc += v2 * x2;
+      acc += v3 * x3;
+    }
+    for (; q < e; q += g) acc += v[q] * xs(ci[q]);
+    for (int off = g >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) f(row, acc);
+  }
+  __syncthreads();
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kTailNT) tail_kernel(TailArgs<T> S) {
+  extern __shared__ unsigned char lds[];
+  auto put = [&](const TailCsr<T>& M) {
+    T* v = reinterpret_cast<T*>(lds + M.o_v);
+    int* rp = reinterpret_cast<int*>(lds + M.o_rp);
+    uint16_t* ci = reinterpret_cast<uint16_t*>(lds + M.o_ci);
+    for (int t = threadIdx.x; t < M.nnz; t += kTailNT) {
+      v[t] = M.v[t];
+      ci[t] = (uint16_t)M.ci[t];
+    }
+    for (int t = threadIdx.x; t <= M.n; t += kTailNT) rp[t] = M.rp[t];
+  };
+  for (int l = 0; l < S.nlev; ++l) {
+    const TailLevel<T>& L = S.lev[l];
+    put(L.A);
+    put(L.P);
+    put(L.R);
+    T* dinv = reinterpret_cast<T*>(lds + L.o_dinv);
+    for (int t = threadIdx.x; t < L.A.n; t += kTailNT) dinv[t] = L.dinv[t];
+  }
+  // f over the rows of a staged matrix times the LDS vector x
+  auto rows = [&](const TailCsr<T>& M, const T* x, auto f) {
+    tail_rows(M.n, M.lg, reinterpret_cast<const int*>(lds + M.o_rp), reinterpret_cast<const uint16_t*>(lds + M.o_ci),
+              reinterpret_cast<const T*>(lds + M.o_v), [=](int j) { return x[j]; }, f);
+  };
+  // level l's x, t, b, d, r; the coarsest level's x and b
+  enum { VX = 0, VT = 1, VB = 2, VD = 3, VR = 4 };
+  auto vec = [&](int l, int which) { return reinterpret_cast<T*>(lds + S.lev[l].o_vec) + which * S.lev[l].A.n; };
+  T* const cx = reinterpret_cast<T*>(lds + S.o_coarse);
+  T* const cb = cx + S.nc;
+  {
+    T* b = S.nlev > 0 ? vec(0, VB) : cb;
+    const T* r = S.r;
+    tail_rows(S.R.n, S.R.lg, S.R.rp, S.R.ci, S.R.v, [=](int j) { return r[j]; }, [=](int row, T a) { b[row] = a; });
+  }
+  // one smoother step: xo = x + its correction, d updated
+  auto smooth = [&](const TailLevel<T>& L, const T* x, T* xo, const T* b, T* d, T c1, T c2) {
+    const T* dinv = reinterpret_cast<const T*>(lds + L.o_dinv);
+    const int type = S.type;
+    rows(L.A, x, [=](int row, T a) {
+      if (type == 0) {
+        xo[row] = x[row] + c1 * dinv[row] * (b[row] - a);
+      } else {
+        const T r = dinv[row] * (b[row] - a);
+        const T dn = (c1 != T(0) ? c1 * d[row] : T(0)) + c2 * r;
+        d[row] = dn;
+        xo[row] = x[row] + dn;
+      }
+    });
+  };
+  const int moves = S.npre > 1 ? S.npre - 1 : 0;  // steps that move x to t or back before the correction
+  for (int l = 0; l < S.nlev; ++l) {
+    const TailLevel<T>& L = S.lev[l];
+    T *x = vec(l, VX), *t = vec(l, VT), *b = vec(l, VB), *d = vec(l, VD), *r = vec(l, VR);
+    const T* dinv = reinterpret_cast<const T*>(lds + L.o_dinv);
+    for (int i = threadIdx.x; i < L.A.n; i += kTailNT) {
+      const T v = S.npre > 0 ? L.c0 * dinv[i] * b[i] : T(0);
+      x[i] = v;
+      d[i] = v;
+    }
+    __syncthreads();
+    for (int st = 1; st <= moves; ++st) {
+      smooth(L, x, t, b, d, L.pre1[st], L.pre2[st]);
+      T* w = x; x = t; t = w;
+    }
+    rows(L.A, x, [=](int row, T a) { r[row] = b[row] - a; });
+    T* bn = l + 1 < S.nlev ? vec(l + 1, VB) : cb;
+    rows(L.R, r, [=](int row, T a) { bn[row] = a; });
+  }
+  // coarsest level: FP64 sums in every precision, a wavefront per row
+  {
+    constexpr int kRows = (int)kTailCoarse / (kTailNT / 64);  // rows of a wavefront, loaded together
+    const int j = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double acc[kRows];
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+      const int row = wave + i * (kTailNT / 64);
+      acc[i] = row < S.nc && j < S.nc ? S.cinv[(int64_t)row * S.nc + j] * (double)cb[j] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+      const int row = wave + i * (kTailNT / 64);
+      const double sum = wave_sum(acc[i]);
+      if (row < S.nc && j == 0) {
+        cx[row] = (T)sum;
+        if (S.nlev == 0) S.x[row] = (T)sum;
+      }
+    }
+    __syncthreads();
+  }
+  for (int l = S.nlev - 1; l >= 0; --l) {
+    const TailLevel<T>& L = S.lev[l];
+    T *x = vec(l, (moves & 1) ? VT : VX), *t = vec(l, (moves & 1) ? VX : VT), *b = vec(l, VB), *d = vec(l, VD);
+    const T* xc = l + 1 < S.nlev ? vec(l + 1, ((moves + S.npost) & 1) ? VT : VX) : cx;
+    rows(L.P, xc, [=](int row, T a) { x[row] += a; });
+    for (int st = 0; st < S.npost; ++st) {
+      smooth(L, x, t, b, d, L.post1[st], L.post2[st]);
+      T* w = x; x = t; t = w;
+    }
+    if (l == 0)
+      for (int i = threadIdx.x; i < L.A.n; i += kTailNT) S.x[i] = x[i];
+  }
+}
+
+// lanes per row: the block's threads over the rows, at least one entry a lane
+template <typename T>
+TailCsr<T> tail_csr(const Csr& M) {
+  const double avg = M.n ? (double)M.nnz / (double)M.n : 1.0;
+  int lg = 0;
+  while (lg < 6 && (M.n << (lg + 1)) <= kTailNT && avg > (double)(1 << lg)) ++lg;
+  return TailCsr<T>{M.rp.get(), M.ci.get(), vals_of<T>(M), (int)M.n, (int)M.nnz, lg, 0, 0, 0};
+}
+
+// Arguments of the tail from level l (R: the restriction into it); returns its
+// LDS bytes, 0 when the levels do not fit.
+template <typename T>
+size_t plan_tail(const Handle& h, int l, const Csr& R, TailArgs<T>& S) {
+  const Hierarchy& H = h.H;
+  S.nlev = H.coarse - l;
+  S.type = h.prm.smootherType;
+  S.npre = h.prm.preInnerIters;
+  S.npost = h.prm.postInnerIters * (h.prm.postRelaxes > 0 ? h.prm.postRelaxes : 1);
+  if (l < 1 || S.nlev < 0 || S.nlev > kTailLevels || S.npre > kTailSteps || S.npost > kTailSteps) return 0;
+  if (R.nnz > kTailRnnz || H.nc > kTailCoarse) return 0;
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at = (at + bytes + 15) & ~(size_t)15;
+    return (int)o;
+  };
+  S.nc = (int)H.nc;
+  S.o_coarse = take(2 * sizeof(T) * (size_t)H.nc);
+  auto place = [&](const Csr& M) {
+    TailCsr<T> c = tail_csr<T>(M);
+    c.o_v = take(sizeof(T) * (size_t)M.nnz);
+    c.o_rp = take(sizeof(int) * (size_t)(M.n + 1));
+    c.o_ci = take(sizeof(uint16_t) * (size_t)M.nnz);
+    return c;
+  };
+  for (int j = l; j < H.coarse; ++j) {
+    const Level& L = *H.levels[j];
+    if (L.A.n > kTailRows || L.A.nnz * (int64_t)sizeof(T) > (int64_t)kTailLds) return 0;
+    TailLevel<T>& t = S.lev[j - l];
+    t.A = place(L.A);
+    t.P = place(L.P);
+    t.R = place(L.R);
+    t.dinv = dinv_of<T>(L);
+    t.o_dinv = take(sizeof(T) * (size_t)L.A.n);
+    t.o_vec = take(5 * sizeof(T) * (size_t)L.A.n);
+    if (at > kTailLds) return 0;
+    const Smoother sm = smoother_for(h, L);
+    ChebSeq a(sm), b(sm);
+    t.c0 = (T)(sm.type ? 1.0 / a.theta : sm.omega);
+    for (int st = 0; st < kTailSteps; ++st) {
+      double c1 = sm.omega, c2 = 0.0;
+      if (sm.type) a.next(st, c1, c2);
+      t.pre1[st] = (T)c1;
+      t.pre2[st] = (T)c2;
+      c1 = sm.omega;
+      c2 = 0.0;
+      if (sm.type) b.next(st, c1, c2);
+      t.post1[st] = (T)c1;
+      t.post2[st] = (T)c2;
+    }
+  }
+  S.R = tail_csr<T>(R);
+  S.cinv = H.cinv64.get();
+  return at;
+}
+
 // Cycle types (cycleType): 0 V; 1 W, whose coarse correction is two W-cycles
 // of the next level, the second from the first's result (cycles/wcycle.h);
 // 2 F, whose coarse correction is an F-cycle of the next level followed by a
@@ -1113,6 +1381,24 @@ T* coarse_correction(Handle& h, int l, int k, bool next_first, int type) {
   if (type != kCycleV && l + 1 != h.H.coarse)
     xc = vcycle<T>(h, l + 1, LV<T>::b(N), k, nullptr, false, type == kCycleW ? kCycleW : kCycleV, xc);
   return xc;
+}
+
+// Level l's coarse correction from its residual r: restriction by R and the
+// cycle of level l+1, in one launch where the levels below are small
+template <typename T>
+T* correction(Handle& h, int l, const Csr& R, const T* r, int k, int type) {
+  if (k == 1 && type == kCycleV) {
+    TailArgs<T> S{};
+    if (const size_t bytes = plan_tail<T>(h, l + 1, R, S)) {
+      S.r = r;
+      S.x = LV<T>::x(*h.H.levels[l + 1]);
+      tail_kernel<T><<<1, kTailNT, bytes, h.stream>>>(S);
+      HIP_LAUNCH_CHECK();
+      return S.x;
+    }
+  }
+  const bool next_first = restrict_first<T>(h, l, R, r, k);
+  return coarse_correction<T>(h, l, k, next_first, type);
 }
 
 // One cycle of the given type on level l for the right-hand side b (level l
@@ -1143,30 +1429,11 @@ T* vcycle(Handle& h, int l, const T* b, int k, Level0Io* io, bool first_done, in
     ProfScope ps(h, (h.profiling && l == 0) ? "resid_l0" : "", matrix_bytes<T>(A, k) + 3.0 * A.n * k * sizeof(T));
     spmv_op<T, kResid>(A, k, cur, r, b, (const T*)nullptr, nullptr, nullptr, T(0), T(0), s);
   }
-  const bool next_first = restrict_first<T>(h, l, L.R, r, k);
-  T* xc = coarse_correction<T>(h, l, k, next_first, type);
+  T* xc = correction<T>(h, l, L.R, r, k, type);
   spmv_op<T, kAdd>(L.P, k, xc, cur, nullptr, (const T*)nullptr, nullptr, nullptr, T(0), T(0), s);
   cur = smooth<T>(h, l, A, b, cur, oth, d, nu_post, false, k, io);
   return cur;
 }
-
-// Chebyshev coefficients of step `step` of a smoother on [lmin, lmax]
-struct ChebSeq {
-  double theta, delta, sigma, rho_old;
-  explicit ChebSeq(const Smoother& S)
-      : theta(0.5 * (S.lmax + S.lmin)), delta(0.5 * (S.lmax - S.lmin)), sigma(theta / delta), rho_old(delta / theta) {}
-  void next(int step, double& c1, double& c2) {
-    if (step == 0) {
-      c1 = 0.0;
-      c2 = 1.0 / theta;
-    } else {
-      const double rho_new = 1.0 / (2.0 * sigma - rho_old);
-      c1 = rho_new * rho_old;
-      c2 = 2.0 * rho_new / delta;
-      rho_old = rho_new;
-    }
-  }
-};
 
 // Precision 2, one column: the level-0 part of the V-cycle in y = D^1/2 x (the
 // same V-cycle as the FP32 one: Chebyshev/Jacobi on a matrix similar to
@@ -1246,8 +1513,7 @@ unsigned vcycle0_half(Handle& h, const double* r64, double* z64, double* partial
     sell_half_kernel<kResid><<<g, kNT, 0, s>>>(n, O.nslices, V, O.sh.get(), H.ah_diag.get(), cur, bh, rr, nullptr,
                                                 nullptr, 0.0f, 0.0f);
   HIP_LAUNCH_CHECK();
-  const bool next_first = restrict_first<float>(h, 0, H.rh, rr, 1);
-  float* xc = coarse_correction<float>(h, 0, 1, next_first, cycle_type(h));
+  float* xc = correction<float>(h, 0, H.rh, rr, 1, cycle_type(h));
   spmv_op<float, kAdd>(H.ph, 1, xc, cur, nullptr, (const float*)nullptr, nullptr, nullptr, 0.0f, 0.0f, s);
   // post-smoothing; the last step writes z and the r.z partials
   ChebSeq cp(S);
