@@ -129,28 +129,31 @@ struct SpmvRow {
     if (MODE == kAdd) y = yp[row];
   }
 
-  template <int MODE>
-  __device__ __forceinline__ void store(int64_t row, T acc, T* __restrict__ yp, T* __restrict__ dp,
-                                        T* __restrict__ xn, T c1, T c2) {
+  // returns the row's result; LAST: a smoother's last step, d is not needed
+  template <int MODE, bool LAST = false>
+  __device__ __forceinline__ T store(int64_t row, T acc, T* __restrict__ yp, T* __restrict__ dp,
+                                     T* __restrict__ xn, T c1, T c2) {
+    T out = acc;
     if (MODE == kAssign) {
-      yp[row] = acc;
+      yp[row] = out;
     } else if (MODE == kAssignScale) {
       yp[row] = acc;
-      const T v = c1 * dinv * acc;
-      xn[row] = v;
-      if (dp) dp[row] = v;
+      out = c1 * dinv * acc;
+      xn[row] = out;
+      if (dp) dp[row] = out;
     } else if (MODE == kResid) {
-      yp[row] = b - acc;
+      yp[row] = out = b - acc;
     } else if (MODE == kAdd) {
-      yp[row] = y + acc;
+      yp[row] = out = y + acc;
     } else if (MODE == kJacobi) {
-      xn[row] = x + c1 * dinv * (b - acc);
+      xn[row] = out = x + c1 * dinv * (b - acc);
     } else {
       const T r = dinv * (b - acc);
       const T dn = (c1 != T(0) ? c1 * d : T(0)) + c2 * r;
-      dp[row] = dn;
-      xn[row] = x + dn;
+      if (!LAST) dp[row] = dn;
+      xn[row] = out = x + dn;
     }
+    return out;
   }
 };
 

@@ -415,6 +415,39 @@ __global__ void __launch_bounds__(kLdsMaxNT) sell_lds_out_kernel(
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
+// Last level-0 smoothing step of an FP64 V-cycle (one column, staged copy):
+// as sell_lds_kernel, with per-block partials of b.xn = r.z for the PCG beta and
+// without the write of d.  A dot product of its own is one more launch and
+// reads r and z again: 49^3 7.2 + 3.9 us for the two, 7.4 here; 65^2 3.9 + 2.9
+// and 4.3 (solves, with the first step in the update: 49^3 3.49 -> 3.36 ms,
+// 65^2 1.86 -> 1.77, 12^3 1.31 -> 1.24, 131 x 150 x 119 30.9 -> 30.5).
+template <int MODE, int HEAD>
+__global__ void __launch_bounds__(kLdsMaxNT) sell_lds_rz_kernel(
+    int64_t n, int64_t nslices, SellView S, LdsView L, const double* __restrict__ sv, const double* __restrict__ x,
+    const double* __restrict__ b, const double* __restrict__ dinv, double* __restrict__ d, double* __restrict__ xn,
+    double c1, double c2, double* __restrict__ partials) {
+  extern __shared__ unsigned char lds_raw[];
+  double* xs = reinterpret_cast<double*>(lds_raw);
+  __shared__ double s_buf[kLdsMaxNT / 64];
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const LdsWave w = lds_wave(L, blk, n, nslices);
+  LdsStage G;
+  SliceHead<double, HEAD> H;
+  SpmvRow<double> R;
+  G.begin(L, blk);
+  if (w.live) lds_head(H, S, L, w.slice, w.lane, sv);
+  if (w.on) R.template load<MODE>(w.pos, S.sd64, x, nullptr, b, dinv, d, c1);
+  G.finish<double>(L, x, xs);
+  double part = 0.0;
+  if (w.on) {
+    double acc = lds_row_sum<double>(H, L, w.lane, sv, xs);
+    if (S.sd64) acc += R.sd * R.x;  // the diagonal term, last
+    part = R.b * R.template store<MODE, true>(w.pos, acc, nullptr, nullptr, xn, c1, c2);
+  }
+  const double tot = block_sum(part, s_buf, blockDim.x >> 6);
+  if (threadIdx.x == 0) partials[blockIdx.x] = tot;
+}
+
 // ---- precision 2: level-0 smoothing in y = D^1/2 x on D^-1/2 A D^-1/2 with
 // FP16 off-diagonals (diagonal 1 + eps_i held apart in FP32)
 
@@ -691,14 +724,17 @@ __global__ void __launch_bounds__(kLdsMaxNT) pcg_sell_lds_dot_kernel(
 }
 
 // x += alpha p; r -= alpha q; partials of r.r
-// (and r32 = fl32(r), the FP32 V-cycle's input, when r32 is given)
-template <int KP>
+// (and bt = fl(r), the FP32 V-cycle's right-hand side, when bt is given; with
+// x0 the level-0 smoother's first step from zero on it, or on r itself in an
+// FP64 V-cycle: at 131 x 150 x 119 18.6 us and 15.4 us for that step by itself,
+// 29.7 us together; 65^2 2.9 and 2.1 us, 3.0 together)
+template <int KP, typename T>
 __global__ void __launch_bounds__(kNT) pcg_update_kernel(int64_t n, int k, double* __restrict__ x,
                                                        double* __restrict__ r, const double* __restrict__ p,
                                                        const double* __restrict__ q, double* __restrict__ partials,
-                                                       const double* __restrict__ scal, float* __restrict__ r32,
-                                                       const float* __restrict__ dinv32, float* __restrict__ x0,
-                                                       float* __restrict__ d0, float c0) {
+                                                       const double* __restrict__ scal, T* __restrict__ bt,
+                                                       const T* __restrict__ dinv, T* __restrict__ x0,
+                                                       T* __restrict__ d0, T c0) {
   __shared__ double s_buf[kNT];
   double part = 0.0;
   const int c = threadIdx.x & (KP - 1);
@@ -710,14 +746,11 @@ __global__ void __launch_bounds__(kNT) pcg_update_kernel(int64_t n, int k, doubl
       x[t] += a * p[t];
       double rv = r[t] - a * q[t];
       r[t] = rv;
-      if (r32) {
-        const float bv = (float)rv;
-        r32[t] = bv;
-        if (x0) {  // the level-0 smoother's first step from zero on fl32(r)
-          const float v = c0 * dinv32[row] * bv;
-          x0[t] = v;
-          if (d0) d0[t] = v;
-        }
+      if (bt) bt[t] = (T)rv;
+      if (x0) {  // the level-0 smoother's first step from zero
+        const T v = c0 * dinv[row] * (T)rv;
+        x0[t] = v;
+        if (d0) d0[t] = v;
       }
       part += rv * rv;
     }
@@ -925,17 +958,23 @@ bool fused_out(const Level0Io* io, const Csr& A, int k) {
 }
 
 // The last level-0 smoothing step for k > 1 columns with r.z partials
-// (io->r64 and io->partials, no io->z64) on the FP32 staged copy
+// (io->r64 and io->partials, no io->z64) on the staged copy
 template <typename T>
 bool multi_out(const Level0Io* io, const Csr& A, int k) {
-  return std::is_same<T, float>::value && io && io->r64 && io->partials && !io->z64 && k <= 64 &&
-         multi_staged<float>(A, k) && A.srow.size() == 0;
+  return io && io->r64 && io->partials && !io->z64 && k > 1 && k <= 64 && multi_staged<T>(A, k) && A.srow.size() == 0;
+}
+
+// The same for one column of an FP64 V-cycle
+template <typename T>
+bool rz_out(const Level0Io* io, const Csr& A, int k) {
+  return std::is_same<T, double>::value && io && io->partials && k == 1 && A.nslices > 0 && A.s64.size() > 0 &&
+         A.lds.bs > 0 && A.srow.size() == 0;
 }
 
 // nu steps of the smoother from x = 0 (zero == true) or from the given x.
 // Buffers x and t ping-pong; returns the buffer that holds the result (with
 // io->z64 set, the last step writes there instead and nullptr is returned;
-// with multi_out, the last step also writes the r.z partials).
+// with multi_out and rz_out, the last step also writes the r.z partials).
 // first_done: the first step from zero is already in x (and d), taken by the
 // restriction that produced b.
 template <typename T>
@@ -959,6 +998,7 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
   const bool in64 = zero && io && io->r64 && std::is_same<T, float>::value && k == 1;
   const bool out64 = !zero && fused_out<T>(io, A, k);
   const bool outk = !zero && multi_out<T>(io, A, k);
+  const bool outrz = !zero && rz_out<T>(io, A, k);
   auto first_step = [&](T* xo, T* dout, double c) {
     if (in64) {
       scale_in_kernel<<<grid_for(A.n, 256), 256, 0, s>>>(A.n, (const float*)dinv, io->r64, io->b32, (float*)xo,
@@ -997,6 +1037,20 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
     HIP_LAUNCH_CHECK();
     io->nb = g;
   };
+  // the last step into xn with the r.z partials (outk, outrz)
+  auto last_rz = [&](auto mode, const T* cur, T* xn, double c1, double c2) {
+    if (outk) {
+      launch_lds_multi<T, mode.value, 2>(A, k, cur, nullptr, b, dinv, d, xn, (T)c1, (T)c2, io->r64, io->partials, s);
+      io->nb = multi_blocks(A);
+    } else if constexpr (std::is_same<T, double>::value) {
+      lds_launch(A, sizeof(T), [&](auto head, unsigned nb, unsigned nt) {
+        sell_lds_rz_kernel<mode.value, head.value><<<nb, nt, sizeof(T) * (size_t)A.lds.maxc, s>>>(
+            A.n, A.nslices, sell_view(A), lds_view(A.lds), A.s64.get(), cur, b, dinv, d, xn, c1, c2, io->partials);
+        io->nb = nb;
+      });
+    }
+    HIP_LAUNCH_CHECK();
+  };
   T* cur = x;
   T* nxt = t;
   int step = 0;
@@ -1012,16 +1066,11 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
         last_step(kJacobi, cur, S.omega, 0.0);
         return nullptr;
       }
-      if constexpr (std::is_same<T, float>::value) {
-        if (outk && step == nu - 1) {
-          launch_lds_multi<float, kJacobi, 2>(A, k, cur, nullptr, b, dinv, nullptr, nxt, (float)S.omega, 0.0f, io->r64,
-                                              io->partials, s);
-          HIP_LAUNCH_CHECK();
-          io->nb = multi_blocks(A);
-          return nxt;
-        }
-      }
       ProfScope ps(h, prof ? "smooth_l0" : "", sweep_bytes);
+      if ((outk || outrz) && step == nu - 1) {
+        last_rz(std::integral_constant<int, kJacobi>{}, cur, nxt, S.omega, 0.0);
+        return nxt;
+      }
       spmv_op<T, kJacobi>(A, k, cur, nullptr, b, dinv, nullptr, nxt, w, T(0), s);
       T* tmp = cur; cur = nxt; nxt = tmp;
     }
@@ -1051,16 +1100,11 @@ T* smooth(Handle& h, int l, const Csr& A, const T* b, T* x, T* t, T* d, int nu, 
       last_step(kCheb, cur, c1, c2);
       return nullptr;
     }
-    if constexpr (std::is_same<T, float>::value) {
-      if (outk && step == nu - 1) {
-        launch_lds_multi<float, kCheb, 2>(A, k, cur, nullptr, b, dinv, d, nxt, (float)c1, (float)c2, io->r64,
-                                          io->partials, s);
-        HIP_LAUNCH_CHECK();
-        io->nb = multi_blocks(A);
-        return nxt;
-      }
-    }
     ProfScope ps(h, prof ? "smooth_l0" : "", sweep_bytes);
+    if ((outk || outrz) && step == nu - 1) {
+      last_rz(std::integral_constant<int, kCheb>{}, cur, nxt, c1, c2);
+      return nxt;
+    }
     spmv_op<T, kCheb>(A, k, cur, nullptr, b, dinv, d, nxt, (T)c1, (T)c2, s);
     T* tmp = cur; cur = nxt; nxt = tmp;
   }
@@ -1124,8 +1168,10 @@ constexpr size_t kTailLds = 150 * 1024;
 // use the whole chip)
 constexpr int64_t kTailRnnz = 16384;
 constexpr int64_t kTailCoarse = 64;
-// rows of a smoothed level: 475 rows break even (300 x 280: 4.94 -> 4.89 ms a
-// solve), 689 lose (379 x 321: 4.97 -> 5.19 ms), 271 gain (71 x 55: 2.07 -> 1.80)
+// rows of a smoothed level: 260 x 240 FP64 solves in 4.39 ms with its
+// level of 250 to 480 rows in here, 4.90 with it in launches; larger ones mostly fall to
+// the restriction's limit above (a limit of 1024 rows times the same from 300 x
+// 280 to 500 x 480, 13^3 to 49^3)
 constexpr int64_t kTailRows = 480;
 
 template <typename T>
@@ -1555,48 +1601,51 @@ struct PrecOut {
 // correction, sliced ELL: the FP64 <-> FP32 conversions are fused into the
 // first and last level-0 smoothing steps, and the last one also writes
 // per-block partials of r.z.
-struct First0 {
-  bool on = false;
-  float* b32 = nullptr;
-  const float* dinv = nullptr;
-  float* x0 = nullptr;
-  float* d0 = nullptr;
-  float c0 = 0.0f;
-};
-
 bool fused_level0(const Handle& h, int k, bool partials) {
   const int nu_post = h.prm.postInnerIters * (h.prm.postRelaxes > 0 ? h.prm.postRelaxes : 1);
   return partials && h.H.precision >= 1 && k == 1 && h.H.coarse > 0 && h.prm.preInnerIters >= 1 && nu_post >= 1 &&
          h.A.nslices > 0 && h.A.s32.size() > 0 && h.A.sell_g == 1;
 }
 
-// Outputs of the PCG update for an FP32 level-0 V-cycle: b32 = fl32(r), and
-// the smoother's first step from zero, x0 = c0 dinv b32 (and d0 = x0 for
-// Chebyshev).  Off for the FP16 level-0 smoother (its own first step) and for
-// hierarchies without level-0 smoothing.
-First0 first0_for(Handle& h, int k) {
-  First0 f;
-  if (h.H.precision < 1 || h.H.coarse <= 0 || h.prm.preInnerIters < 1) return f;
+// Outputs of the PCG update for a level-0 V-cycle in T: b = fl32(r) (FP32; an
+// FP64 V-cycle reads r), and the smoother's first step from zero, x0 = c0 dinv
+// b (and d0 = x0 for Chebyshev).  Off for the FP16 level-0 smoother (its own
+// first step) and for hierarchies without level-0 smoothing.
+template <typename T>
+struct First0 {
+  bool on = false;
+  T* b = nullptr;
+  const T* dinv = nullptr;
+  T* x0 = nullptr;
+  T* d0 = nullptr;
+  T c0 = T(0);
+};
+
+template <typename T>
+First0<T> first0_for(Handle& h, int k) {
+  constexpr bool f32 = std::is_same<T, float>::value;
+  First0<T> f;
+  if ((h.H.precision >= 1) != f32 || h.H.coarse <= 0 || h.prm.preInnerIters < 1) return f;
   if (h.H.precision == 2 && fused_level0(h, k, true) && h.H.ah.nslices > 0) return f;
   Level& L0 = *h.H.levels[0];
   const Smoother S = smoother_for(h, L0);
-  f.b32 = L0.b32.get();
-  f.dinv = L0.dinv32.get();
-  f.x0 = L0.x32.get();
+  if (f32) f.b = LV<T>::b(L0);
+  f.dinv = dinv_of<T>(L0);
+  f.x0 = LV<T>::x(L0);
   if (S.type == 0) {
-    f.c0 = (float)S.omega;
+    f.c0 = (T)S.omega;
   } else {
-    f.c0 = (float)(1.0 / (0.5 * (S.lmax + S.lmin)));
-    f.d0 = L0.d32.get();
+    f.c0 = (T)(1.0 / (0.5 * (S.lmax + S.lmin)));
+    f.d0 = LV<T>::d(L0);
   }
   f.on = f.dinv != nullptr && f.x0 != nullptr;
-  return f;
+  return f.on ? f : First0<T>();
 }
 
 // z = M r at level 0 (FP64 r); k columns.  z is written only on the fused
 // path; otherwise it is left where the V-cycle put it (no copy).  r32_ready:
-// the level-0 FP32 right-hand side already holds fl32(r); first_ready: and
-// the level-0 smoother's first step from zero is in its x (and d).
+// the level-0 FP32 right-hand side already holds fl32(r); first_ready: the
+// level-0 smoother's first step from zero is in its x (and d) too.
 PrecOut precondition_pcg(Handle& h, const double* r, double* z, int k, double* partials, bool r32_ready,
                          bool first_ready) {
   hipStream_t s = h.stream;
@@ -1605,7 +1654,13 @@ PrecOut precondition_pcg(Handle& h, const double* r, double* z, int k, double* p
   PrecOut o;
   const int type = cycle_type(h);
   if (h.H.precision == 0) {
-    o.z64 = vcycle<double>(h, 0, r, k, nullptr, false, type);
+    // the last level-0 smoothing step also writes the r.z partials when it
+    // runs on the staged copy (o.nb stays 0 otherwise)
+    Level0Io io;
+    io.r64 = r;
+    io.partials = partials;
+    o.z64 = vcycle<double>(h, 0, r, k, partials ? &io : nullptr, first_ready, type);
+    o.nb = io.nb;
     return o;
   }
   if (fused_level0(h, k, partials != nullptr)) {
@@ -1941,30 +1996,29 @@ void dot(Handle& h, int k, const double* a, const B* b, int mode, int slot) {
   }
 }
 
-template <int KP>
-void launch_update(Handle& h, int k, double tol2, float* r32, const First0* f0) {
+template <int KP, typename T>
+void launch_update(Handle& h, int k, double tol2, const First0<T>& f0) {
   const int64_t n = h.A.n;
   unsigned g = vec_grid(n, KP);
-  pcg_update_kernel<KP><<<g, kNT, 0, h.stream>>>(n, k, h.kx.get(), h.kr.get(), h.kp.get(), h.kq.get(),
-                                                 h.partials.get(), h.scal.get(), f0 ? f0->b32 : r32,
-                                                 f0 ? f0->dinv : nullptr, f0 ? f0->x0 : nullptr,
-                                                 f0 ? f0->d0 : nullptr, f0 ? f0->c0 : 0.0f);
+  pcg_update_kernel<KP, T><<<g, kNT, 0, h.stream>>>(n, k, h.kx.get(), h.kr.get(), h.kp.get(), h.kq.get(),
+                                                    h.partials.get(), h.scal.get(), f0.b, f0.dinv, f0.x0, f0.d0,
+                                                    f0.c0);
   HIP_LAUNCH_CHECK();
   finish(h, (int)g, k, F_RR, 0, tol2);
 }
 
-// x += alpha p, r -= alpha q, |r|^2, and r32 = fl32(r) when r32 is given
-// (with f0: fl32(r) into the level-0 right-hand side and the smoother's first
-// step from zero into its x and d)
-void update(Handle& h, int k, double tol2, float* r32, const First0* f0 = nullptr) {
+// x += alpha p, r -= alpha q, |r|^2, and what f0 names: fl32(r) into the
+// level-0 right-hand side, the smoother's first step from zero into its x and d
+template <typename T>
+void update(Handle& h, int k, double tol2, const First0<T>& f0) {
   switch (pow2_at_least(k)) {
-    case 1: launch_update<1>(h, k, tol2, r32, f0); break;
-    case 2: launch_update<2>(h, k, tol2, r32, f0); break;
-    case 4: launch_update<4>(h, k, tol2, r32, f0); break;
-    case 8: launch_update<8>(h, k, tol2, r32, f0); break;
-    case 16: launch_update<16>(h, k, tol2, r32, f0); break;
-    case 32: launch_update<32>(h, k, tol2, r32, f0); break;
-    default: launch_update<64>(h, k, tol2, r32, f0); break;
+    case 1: launch_update<1, T>(h, k, tol2, f0); break;
+    case 2: launch_update<2, T>(h, k, tol2, f0); break;
+    case 4: launch_update<4, T>(h, k, tol2, f0); break;
+    case 8: launch_update<8, T>(h, k, tol2, f0); break;
+    case 16: launch_update<16, T>(h, k, tol2, f0); break;
+    case 32: launch_update<32, T>(h, k, tol2, f0); break;
+    default: launch_update<64, T>(h, k, tol2, f0); break;
   }
 }
 
@@ -2145,17 +2199,22 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
       }
     } ev_guard{evs};
     int restarts = 0;
-    // the unfused mixed-precision V-cycle takes fl32(r), written by the update
-    float* r32 = (h.H.precision >= 1 && !fused_level0(h, k, true)) ? h.H.levels[0]->b32.get() : nullptr;
-    // and the level-0 smoother's first step from zero (with fl32(r) on the
-    // fused path) comes from the update as well
-    const First0 f0 = first0_for(h, k);
+    // the level-0 smoother's first step from zero (on fl32(r) in the mixed
+    // precisions) comes from the update; an unfused mixed-precision V-cycle
+    // without one still takes fl32(r)
+    First0<float> f32 = first0_for<float>(h, k);
+    const First0<double> f64 = first0_for<double>(h, k);
+    if (!f32.on && h.H.precision >= 1 && !fused_level0(h, k, true)) f32.b = h.H.levels[0]->b32.get();
+    auto update_all = [&]() {  // x, r, rr, act
+      if (f64.on) update<double>(h, k, tol2, f64);
+      else update<float>(h, k, tol2, f32);
+    };
     while (any) {
       // z = M r and rz = r.z (fused into the last level-0 smoothing step when
       // possible); z stays where the preconditioner left it
       auto precondition_dot = [&](int mode, int slot, bool r32_ready) {
         const PrecOut o = precondition_pcg(h, h.kr.get(), h.kz.get(), k, h.partials.get(),
-                                           r32_ready && (r32 || f0.on), r32_ready && f0.on);
+                                           r32_ready && f32.b, r32_ready && (f32.on || f64.on));
         if (o.nb) finish(h, (int)o.nb, k, mode, slot);
         else if (o.z32) dot(h, k, h.kr.get(), o.z32, mode, slot);
         else dot(h, k, h.kr.get(), o.z64, mode, slot);
@@ -2183,7 +2242,7 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
           pcg_p_kernel<double><<<grid_for(m, 256), 256, 0, s>>>(m, k, o.z64, h.kp.get(), h.scal.get());
         HIP_LAUNCH_CHECK();
         spmv_dot(h, k);           // q = A p, alpha
-        update(h, k, tol2, r32, f0.on ? &f0 : nullptr);  // x, r, rr, act
+        update_all();
       };
       // Iteration n ends with the n-th |r|^2 finish of this solve; the host
       // reads its record while iteration n + 1 may already run: the next
@@ -2195,7 +2254,7 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
       auto issue = [&](bool first) {
         if (first) {
           spmv_dot(h, k);
-          update(h, k, tol2, r32, f0.on ? &f0 : nullptr);
+          update_all();
         } else {
           run_iteration(h, k, tol2, iteration);
         }
