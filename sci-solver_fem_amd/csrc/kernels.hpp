@@ -158,7 +158,11 @@ struct SpmvRow {
 };
 
 // Single right-hand side: G lanes per row, strided over the row's entries,
-// reduced by a butterfly (fixed order).
+// reduced by a butterfly (fixed order).  A lane's entries go in batches of four
+// (two dependent waits on memory for four entries instead of for each): 49^3
+// FP64 level 1 (5,500 rows, Chebyshev) 4.4 -> 3.4 us, its restriction (200 rows)
+// 8.3 -> 4.7; 161^3 FP32 level 2 5.6 -> 4.9.
+constexpr int kCsrBatch = 4;
 template <typename V, typename T, int G, int MODE>
 __global__ void __launch_bounds__(kNT) csr_vec_kernel(int64_t n, const int32_t* __restrict__ rp,
                                                     const int32_t* __restrict__ ci, const V* __restrict__ val,
@@ -170,7 +174,23 @@ __global__ void __launch_bounds__(kNT) csr_vec_kernel(int64_t n, const int32_t* 
   if (row >= n) return;
   const int s = rp[row], e = rp[row + 1];
   T acc = T(0);
-  for (int k = s + lane; k < e; k += G) acc += (T)ntload(val + k) * x[ntload(ci + k)];
+  for (int k = s + lane; k < e; k += kCsrBatch * G) {
+    int c[kCsrBatch];
+    T v[kCsrBatch], xv[kCsrBatch];
+#pragma unroll
+    for (int j = 0; j < kCsrBatch; ++j) {
+      if (k + j * G < e) {
+        c[j] = ntload(ci + k + j * G);
+        v[j] = (T)ntload(val + k + j * G);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kCsrBatch; ++j)
+      if (k + j * G < e) xv[j] = x[c[j]];
+#pragma unroll
+    for (int j = 0; j < kCsrBatch; ++j)
+      if (k + j * G < e) acc += v[j] * xv[j];
+  }
 #pragma unroll
   for (int off = G / 2; off > 0; off >>= 1) acc += shfl_xor_t(acc, off, G);
   if (lane == 0) spmv_epilogue<MODE, T, V>(row, row, acc, y, x, b, dinv, d, xn, c1, c2);
@@ -229,6 +249,52 @@ __device__ __forceinline__ float sell_val<float, uint16_t>(const uint16_t* p) {
   return (float)__builtin_bit_cast(_Float16, ntload(p));
 }
 
+// Steps k .. k + N - 1 of a lane's entries added to acc in entry order; steps
+// from w (wave-uniform) on read entry w - 1 again and add nothing, without
+// branches between the loads.
+template <int N, typename T, typename V, typename C, typename Col>
+__device__ __forceinline__ T sell_batch(T acc, int k, int w, const C* __restrict__ cp, const V* __restrict__ vp,
+                                        const T* __restrict__ x, Col& col) {
+  C c[N];
+  T v[N], xv[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int e = 64 * (k + j < w ? k + j : w - 1);
+    c[j] = ntload(cp + e);
+    v[j] = sell_val<T>(vp + e);
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) xv[j] = x[col(c[j])];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const T s = acc + v[j] * xv[j];
+    acc = k + j < w ? s : acc;
+  }
+  return acc;
+}
+
+// Sum of w steps of a lane's entries, in entry order.  A batch is two dependent
+// waits on memory (columns and values, then x) whatever its length, so eight
+// steps share them, the last seven or fewer too.  Against batches of four and
+// single last steps, the row's vector entries loaded after the sum (Chebyshev
+// step): 1003 x 701 levels 1 and 2 (53,610 and 4,000 rows) 7.0 and 7.3 -> 5.0
+// and 5.4 us, 97^3 level 1 (43,000 rows, 4 lanes each) 8.6 -> 6.6 us.  Level-0
+// restrictions in 3D (88 entries a row, 8 lanes) are bound by the lines their
+// gathers touch: 42.0 -> 40.5 us at 161^3.
+constexpr int kSellBatch = 8;
+template <typename T, typename V, typename C, typename Col>
+__device__ __forceinline__ T sell_batches(int w, const C* __restrict__ cp, const V* __restrict__ vp,
+                                          const T* __restrict__ x, Col&& col) {
+  T acc = T(0);
+  int k = 0;
+  for (; k + kSellBatch <= w; k += kSellBatch) acc = sell_batch<kSellBatch, T, V>(acc, k, w, cp, vp, x, col);
+  if (w - k > 4)
+    acc = sell_batch<kSellBatch, T, V>(acc, k, w, cp, vp, x, col);
+  else if (w - k > 0)
+    acc = sell_batch<4, T, V>(acc, k, w, cp, vp, x, col);
+  return acc;
+}
+
 // Row sum of slice `slice` (wave-uniform) for this lane's row.  Compact
 // slices read 2-byte column codes: bits 13-15 select one of the slice's 8
 // window bases, bits 0-12 are the offset.
@@ -238,43 +304,15 @@ __device__ __forceinline__ T sell_row_sum(const SellView& S, int slice, int lane
   const int off = __builtin_amdgcn_readfirstlane(S.sp[slice]);
   const int w = __builtin_amdgcn_readfirstlane((S.sp[slice + 1] - off) >> 6);
   const V* vp = sv + off + lane;
-  T acc = T(0);
   static_assert(kSellWindows == 8, "sell_col selects among 8 windows");
   const int32_t* wp = S.swin + slice * kSellWindows;
   const SellWin W{__builtin_amdgcn_readfirstlane(wp[0]), __builtin_amdgcn_readfirstlane(wp[1]),
                   __builtin_amdgcn_readfirstlane(wp[2]), __builtin_amdgcn_readfirstlane(wp[3]),
                   __builtin_amdgcn_readfirstlane(wp[4]), __builtin_amdgcn_readfirstlane(wp[5]),
                   __builtin_amdgcn_readfirstlane(wp[6]), __builtin_amdgcn_readfirstlane(wp[7])};
-  if (W.b0 >= 0) {
-    const uint16_t* cp = S.sc16 + off + lane;
-    int k = 0;
-    for (; k + 4 <= w; k += 4) {
-      const unsigned c0 = ntload(cp + 64 * k), c1 = ntload(cp + 64 * (k + 1)), c2 = ntload(cp + 64 * (k + 2)),
-                     c3 = ntload(cp + 64 * (k + 3));
-      const T v0 = sell_val<T>(vp + 64 * k), v1 = sell_val<T>(vp + 64 * (k + 1)),
-              v2 = sell_val<T>(vp + 64 * (k + 2)), v3 = sell_val<T>(vp + 64 * (k + 3));
-      acc += v0 * x[sell_col(c0, W)];
-      acc += v1 * x[sell_col(c1, W)];
-      acc += v2 * x[sell_col(c2, W)];
-      acc += v3 * x[sell_col(c3, W)];
-    }
-    for (; k < w; ++k) acc += sell_val<T>(vp + 64 * k) * x[sell_col(ntload(cp + 64 * k), W)];
-  } else {
-    const int32_t* cp = S.sc + off + lane;
-    int k = 0;
-    for (; k + 4 <= w; k += 4) {
-      const int c0 = ntload(cp + 64 * k), c1 = ntload(cp + 64 * (k + 1)), c2 = ntload(cp + 64 * (k + 2)),
-                c3 = ntload(cp + 64 * (k + 3));
-      const T v0 = sell_val<T>(vp + 64 * k), v1 = sell_val<T>(vp + 64 * (k + 1)),
-              v2 = sell_val<T>(vp + 64 * (k + 2)), v3 = sell_val<T>(vp + 64 * (k + 3));
-      acc += v0 * x[c0];
-      acc += v1 * x[c1];
-      acc += v2 * x[c2];
-      acc += v3 * x[c3];
-    }
-    for (; k < w; ++k) acc += sell_val<T>(vp + 64 * k) * x[ntload(cp + 64 * k)];
-  }
-  return acc;
+  if (W.b0 >= 0)
+    return sell_batches<T, V>(w, S.sc16 + off + lane, vp, x, [&](unsigned c) { return sell_col(c, W); });
+  return sell_batches<T, V>(w, S.sc + off + lane, vp, x, [](int c) { return c; });
 }
 
 // ---- LDS-staged sliced ELL (one lane per row, row order) ------------------------
@@ -331,7 +369,10 @@ struct LdsStage {
 // loaded before the staging barrier: they do not depend on x, so their memory
 // latency runs beside the staging's (list offsets -> columns -> x) instead of
 // after it.  In groups of four, and the remainder of a row that ends there;
-// which loads are issued is the same for the whole wavefront.
+// which loads are issued is the same for the whole wavefront.  The steps after
+// the head go in batches of eight.  HEAD kLdsBatch: no head, batches of eight;
+// 0: no head, batches of four (fewest registers).
+constexpr int kLdsBatch = -8;
 template <typename V, int HEAD>
 struct SliceHead {
   unsigned c[HEAD > 0 ? HEAD : 1], rc[3];
@@ -399,7 +440,15 @@ __device__ __forceinline__ T lds_row_sum(const SliceHead<V, HEAD>& H, const LdsV
   }
   const V* vp = sv + H.off + lane;
   const uint16_t* cp = L.lc + H.off + lane;
-  int k = HEAD;
+  if constexpr (HEAD != 0) {
+    auto col = [](unsigned c) { return c; };
+    int k = HEAD > 0 ? HEAD : 0;
+    for (; k + kSellBatch <= H.w; k += kSellBatch)
+      acc = sell_batch<kSellBatch, T, V>(acc, k, H.w, cp, vp, xs, col);
+    if (k < H.w) acc = sell_batch<kSellBatch, T, V>(acc, k, H.w, cp, vp, xs, col);
+    return acc;
+  }
+  int k = 0;
   for (; k + 4 <= H.w; k += 4) {
     unsigned c[4];
     V v[4];
@@ -481,15 +530,22 @@ __global__ void __launch_bounds__(kNT) sell_kernel(int64_t n, int64_t nslices, S
       __builtin_amdgcn_readfirstlane((int)(xcd_block(blockIdx.x, gridDim.x) * (kNT / 64) + (threadIdx.x >> 6)));
   const int lane = threadIdx.x & 63;
   if (slice >= nslices) return;
+  // the row's vector entries are loaded beside the first entries
+  const int64_t pos = (int64_t)slice * (64 / G) + lane / G;
+  const bool on = (G == 1 || (lane & (G - 1)) == 0) && pos < n;
+  const T* sd = sell_diag<T>(S);
+  int64_t row = pos;
+  SpmvRow<T> R;
+  if (on) {
+    if (S.srow) row = S.srow[pos];
+    R.template load<MODE>(row, sd, x, y, b, dinv, d, c1);
+  }
   T acc = sell_row_sum<T>(S, slice, lane, sv, x);
 #pragma unroll
   for (int off = G / 2; off > 0; off >>= 1) acc += shfl_xor_t(acc, off, G);
-  const int64_t pos = (int64_t)slice * (64 / G) + lane / G;
-  if ((G == 1 || (lane & (G - 1)) == 0) && pos < n) {
-    const int64_t row = S.srow ? (int64_t)S.srow[pos] : pos;
-    if (const T* sd = sell_diag<T>(S)) acc += sd[row] * x[row];  // the diagonal term, last
-    spmv_epilogue<MODE, T, T>(row, row, acc, y, x, b, dinv, d, xn, c1, c2);
-  }
+  if (!on) return;
+  if (sd) acc += R.sd * R.x;  // the diagonal term, last
+  R.template store<MODE>(row, acc, y, d, xn, c1, c2);
 }
 
 // k right-hand sides with k a multiple of VW = 16 / sizeof(T): L lanes per

@@ -170,9 +170,11 @@ constexpr int64_t kLdsHeadRow = 20;  // average row length above which no head i
 //  * 161^3 FP32, blocks of 8: 88.5 -> 76.6 us (505 MB: 6.6 TB/s); FP16 alike;
 //  * FP64 in blocks of 8 fills the memory system anyway and loses a
 //    wavefront per SIMD to the registers: 8, 12, 16 head steps give 88.7,
-//    93.8, 85.0 us at 131 x 150 x 119 against 81.6 us without;
+//    93.8, 85.0 us at 131 x 150 x 119 against 81.6 us without, batches of
+//    eight 82.0 against 80.4 in fours;
 //  * rows longer than the head (161^3 level 1, ~46 entries): 16.9 us without,
-//    18.5 with; their blocks of 2 slices stage with four wavefronts;
+//    18.5 with, 15.7 without in batches of eight instead of four; their blocks
+//    of 2 slices stage with four wavefronts;
 //  * 2D operators (~7 entries per row) need 8 steps: 1003 x 701 FP64 operator
 //    + p.q 18.2 -> 13.3 us (15.7 with 16 steps' registers);
 //  * fewer blocks than CUs (65^2: 34): a launch is all latency, and the longer
@@ -182,10 +184,10 @@ void lds_launch(const Csr& A, size_t vsize, Fn&& f) {
   const unsigned nb = (unsigned)((A.nslices + A.lds.bs - 1) / A.lds.bs);
   const unsigned nt = 64u * (unsigned)A.lds.bs;
   const bool lengths = A.srow.size() > 0;  // rows in length order (prolongators)
-  if (nb < 256u || A.nnz > kLdsHeadRow * A.n)
-    f(std::integral_constant<int, 0>{}, nb, nt < 256u ? 256u : nt);
-  else if (A.lds.bs > 2 && vsize == 8)
+  if (A.lds.bs > 2 && vsize == 8)
     f(std::integral_constant<int, 0>{}, nb, nt);
+  else if (nb < 256u || A.nnz > kLdsHeadRow * A.n)
+    f(std::integral_constant<int, kLdsBatch>{}, nb, nt < 256u ? 256u : nt);
   else if (A.nnz <= 8 * A.n && !lengths)
     f(std::integral_constant<int, 8>{}, nb, nt);
   else
