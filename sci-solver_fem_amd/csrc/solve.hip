@@ -725,24 +725,57 @@ __global__ void __launch_bounds__(kLdsMaxNT) pcg_sell_lds_dot_kernel(
   if (threadIdx.x == 0) partials[blockIdx.x] = tot;
 }
 
+// Total of nb <= kFoldParts partials in every thread of the block, the same in
+// every block: a kernel that reads alpha or beta sums the partials itself
+// instead of waiting for a finish launch (one column, at most kFoldRows rows:
+// more blocks would read more partials each).  Two finish
+// launches an iteration less: 65^2 1.73 -> 1.69 ms a solve, 12^3 1.23 -> 1.16,
+// 49^3 FP64 3.04 -> 3.00, 20^3 1.88 -> 1.84, 300 x 280 mixed 4.33 -> 4.25.
+constexpr int kFoldParts = 1024;
+constexpr int64_t kFoldRows = 131072;
+__device__ __forceinline__ double fold_sum(const double* __restrict__ part, int nb, double* s_buf) {
+  __shared__ double s_tot;
+  double v = 0.0;
+#pragma unroll
+  for (int j = 0; j < kFoldParts / kNT; ++j) {
+    const int b = (int)threadIdx.x + j * kNT;
+    if (b < nb) v += part[b];
+  }
+  v = block_sum(v, s_buf);
+  if (threadIdx.x == 0) s_tot = v;
+  __syncthreads();
+  return s_tot;
+}
+
 // x += alpha p; r -= alpha q; partials of r.r
+// (FOLD: one column, alpha from the npq partials of p.q and r.z in slot rz)
 // (and bt = fl(r), the FP32 V-cycle's right-hand side, when bt is given; with
 // x0 the level-0 smoother's first step from zero on it, or on r itself in an
 // FP64 V-cycle: at 131 x 150 x 119 18.6 us and 15.4 us for that step by itself,
 // 29.7 us together; 65^2 2.9 and 2.1 us, 3.0 together)
-template <int KP, typename T>
+template <int KP, typename T, bool FOLD>
 __global__ void __launch_bounds__(kNT) pcg_update_kernel(int64_t n, int k, double* __restrict__ x,
                                                        double* __restrict__ r, const double* __restrict__ p,
                                                        const double* __restrict__ q, double* __restrict__ partials,
-                                                       const double* __restrict__ scal, T* __restrict__ bt,
+                                                       const double* scal, T* __restrict__ bt,
                                                        const T* __restrict__ dinv, T* __restrict__ x0,
-                                                       T* __restrict__ d0, T c0) {
+                                                       T* __restrict__ d0, T c0, const double* __restrict__ pq,
+                                                       int npq, int rz, double* __restrict__ scal_out) {
   __shared__ double s_buf[kNT];
+  double alpha = 0.0;
+  if (FOLD) {
+    const double v = fold_sum(pq, npq, s_buf);
+    alpha = (scal[S_ACT] != 0.0 && v != 0.0) ? scal[rz] / v : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      scal_out[S_PQ] = v;
+      scal_out[S_ALPHA] = alpha;
+    }
+  }
   double part = 0.0;
   const int c = threadIdx.x & (KP - 1);
   const int64_t rows_per_grid = (int64_t)gridDim.x * (kNT / KP);
   if (c < k) {
-    const double a = scal[S_ALPHA * k + c];
+    const double a = FOLD ? alpha : scal[S_ALPHA * k + c];
     for (int64_t row = ((int64_t)blockIdx.x * kNT + threadIdx.x) / KP; row < n; row += rows_per_grid) {
       int64_t t = row * k + c;
       x[t] += a * p[t];
@@ -844,8 +877,9 @@ __global__ void __launch_bounds__(kFinNT) pcg_finish_kernel(int nb, int k, const
     scal[slot * k + c] = v;
   } else if (mode == F_ALPHA) {
     scal[S_PQ * k + c] = v;
-    scal[S_ALPHA * k + c] = (scal[S_ACT * k + c] != 0.0 && v != 0.0) ? scal[S_RZ * k + c] / v : 0.0;
+    scal[S_ALPHA * k + c] = (scal[S_ACT * k + c] != 0.0 && v != 0.0) ? scal[slot * k + c] / v : 0.0;
   } else if (mode == F_RR) {
+    if (slot != S_RZ) scal[S_RZ * k + c] = scal[slot * k + c];  // stored there by pcg_p_kernel
     // |r|^2 finishes are numbered on the device (every column counts its
     // own); record n goes to host record n % 2
     const double seq = scal[S_SEQ * k + c] + 1.0;
@@ -873,7 +907,6 @@ __global__ void __launch_bounds__(kFinNT) pcg_finish_kernel(int nb, int k, const
   }
 }
 
-// p = z + beta p
 // p = z + beta p (z as the preconditioner left it: FP64, or the FP32 V-cycle
 // result, converted exactly)
 template <typename Z>
@@ -883,6 +916,28 @@ __global__ void pcg_p_kernel(int64_t m, int k, const Z* __restrict__ z, double* 
   if (t >= m) return;
   int c = (int)(t % k);
   p[t] = (double)z[t] + scal[S_BETA * k + c] * p[t];
+}
+
+// The same for one column with beta from the nrz partials of r.z; r.z goes to
+// S_RZN (other blocks still read S_RZ), moved by the next |r|^2 finish.
+template <typename Z>
+__global__ void __launch_bounds__(kNT) pcg_p_fold_kernel(int64_t n, const Z* __restrict__ z, double* __restrict__ p,
+                                                       double* scal, const double* __restrict__ parts, int nrz) {
+  __shared__ double s_buf[kNT];
+  const int64_t t = (int64_t)blockIdx.x * kNT + threadIdx.x;
+  double zv = 0.0, pv = 0.0;
+  if (t < n) {
+    zv = (double)z[t];
+    pv = p[t];
+  }
+  const double v = fold_sum(parts, nrz, s_buf);
+  const double rz = scal[S_RZ];
+  const double beta = (scal[S_ACT] != 0.0 && rz != 0.0) ? v / rz : 0.0;
+  if (t == 0) {
+    scal[S_RZN] = v;
+    scal[S_BETA] = beta;
+  }
+  if (t < n) p[t] = zv + beta * pv;
 }
 
 // x[:, c] = 0 for every column c whose bit is set in mask (k <= 64 columns)
@@ -1969,62 +2024,84 @@ void run_iteration(Handle& h, int k, double tol2, Fn&& body) {
   HIP_CHECK(hipGraphLaunch(h.iter_graph, h.stream));
 }
 
-void finish(Handle& h, int nb, int k, int mode, int slot, double tol2 = 0.0) {
-  pcg_finish_kernel<<<(unsigned)k, kFinNT, 0, h.stream>>>(nb, k, h.partials.get(), h.scal.get(), mode, slot, tol2,
+void finish(Handle& h, int nb, int k, int mode, int slot, double tol2 = 0.0, int64_t at = 0) {
+  pcg_finish_kernel<<<(unsigned)k, kFinNT, 0, h.stream>>>(nb, k, h.partials.get() + at, h.scal.get(), mode, slot, tol2,
                                                  mode == F_RR ? h.d_act : nullptr);
   HIP_LAUNCH_CHECK();
 }
 
 template <int KP, typename B>
-void launch_dot(Handle& h, int k, const double* a, const B* b, int mode, int slot) {
+unsigned launch_dot(Handle& h, int k, const double* a, const B* b) {
   const int64_t n = h.A.n;
   unsigned g = vec_grid(n, KP);
   pcg_dot_kernel<KP, B><<<g, kNT, 0, h.stream>>>(n, k, a, b, h.partials.get());
   HIP_LAUNCH_CHECK();
-  finish(h, (int)g, k, mode, slot);
+  return g;
+}
+
+// partials of a.b; returns their count per column
+template <typename B>
+unsigned dot_partials(Handle& h, int k, const double* a, const B* b) {
+  switch (pow2_at_least(k)) {
+    case 1: return launch_dot<1, B>(h, k, a, b);
+    case 2: return launch_dot<2, B>(h, k, a, b);
+    case 4: return launch_dot<4, B>(h, k, a, b);
+    case 8: return launch_dot<8, B>(h, k, a, b);
+    case 16: return launch_dot<16, B>(h, k, a, b);
+    case 32: return launch_dot<32, B>(h, k, a, b);
+    default: return launch_dot<64, B>(h, k, a, b);
+  }
 }
 
 // mode F_STORE: scal[slot] = a.b; F_BETA: beta = a.b / rz, rz = a.b
 template <typename B>
 void dot(Handle& h, int k, const double* a, const B* b, int mode, int slot) {
-  switch (pow2_at_least(k)) {
-    case 1: launch_dot<1, B>(h, k, a, b, mode, slot); break;
-    case 2: launch_dot<2, B>(h, k, a, b, mode, slot); break;
-    case 4: launch_dot<4, B>(h, k, a, b, mode, slot); break;
-    case 8: launch_dot<8, B>(h, k, a, b, mode, slot); break;
-    case 16: launch_dot<16, B>(h, k, a, b, mode, slot); break;
-    case 32: launch_dot<32, B>(h, k, a, b, mode, slot); break;
-    default: launch_dot<64, B>(h, k, a, b, mode, slot); break;
-  }
+  finish(h, (int)dot_partials(h, k, a, b), k, mode, slot);
 }
 
+// whether the kernel that reads alpha or beta sums the nb partials itself
+bool folds(const Handle& h, int k, unsigned nb) { return k == 1 && h.A.n <= kFoldRows && nb <= (unsigned)kFoldParts; }
+
 template <int KP, typename T>
-void launch_update(Handle& h, int k, double tol2, const First0<T>& f0) {
+void launch_update(Handle& h, int k, double tol2, const First0<T>& f0, unsigned npq, int rz) {
   const int64_t n = h.A.n;
   unsigned g = vec_grid(n, KP);
-  pcg_update_kernel<KP, T><<<g, kNT, 0, h.stream>>>(n, k, h.kx.get(), h.kr.get(), h.kp.get(), h.kq.get(),
-                                                    h.partials.get(), h.scal.get(), f0.b, f0.dinv, f0.x0, f0.d0,
-                                                    f0.c0);
+  const bool fold = folds(h, k, npq);
+  if (!fold) finish(h, (int)npq, k, F_ALPHA, rz);
+  // its own partials past those that its blocks read
+  const int64_t at = fold ? kFoldParts : 0;
+  auto go = [&](auto f) {
+    pcg_update_kernel<KP, T, f.value><<<g, kNT, 0, h.stream>>>(
+        n, k, h.kx.get(), h.kr.get(), h.kp.get(), h.kq.get(), h.partials.get() + at, h.scal.get(), f0.b, f0.dinv,
+        f0.x0, f0.d0, f0.c0, h.partials.get(), (int)npq, rz, h.scal.get());
+  };
+  if constexpr (KP == 1) {
+    if (fold) go(std::true_type{});
+    else go(std::false_type{});
+  } else {
+    go(std::false_type{});
+  }
   HIP_LAUNCH_CHECK();
-  finish(h, (int)g, k, F_RR, 0, tol2);
+  finish(h, (int)g, k, F_RR, rz, tol2, at);
 }
 
 // x += alpha p, r -= alpha q, |r|^2, and what f0 names: fl32(r) into the
-// level-0 right-hand side, the smoother's first step from zero into its x and d
+// level-0 right-hand side, the smoother's first step from zero into its x and d;
+// alpha from the npq partials of p.q and r.z in slot rz
 template <typename T>
-void update(Handle& h, int k, double tol2, const First0<T>& f0) {
+void update(Handle& h, int k, double tol2, const First0<T>& f0, unsigned npq, int rz) {
   switch (pow2_at_least(k)) {
-    case 1: launch_update<1, T>(h, k, tol2, f0); break;
-    case 2: launch_update<2, T>(h, k, tol2, f0); break;
-    case 4: launch_update<4, T>(h, k, tol2, f0); break;
-    case 8: launch_update<8, T>(h, k, tol2, f0); break;
-    case 16: launch_update<16, T>(h, k, tol2, f0); break;
-    case 32: launch_update<32, T>(h, k, tol2, f0); break;
-    default: launch_update<64, T>(h, k, tol2, f0); break;
+    case 1: launch_update<1, T>(h, k, tol2, f0, npq, rz); break;
+    case 2: launch_update<2, T>(h, k, tol2, f0, npq, rz); break;
+    case 4: launch_update<4, T>(h, k, tol2, f0, npq, rz); break;
+    case 8: launch_update<8, T>(h, k, tol2, f0, npq, rz); break;
+    case 16: launch_update<16, T>(h, k, tol2, f0, npq, rz); break;
+    case 32: launch_update<32, T>(h, k, tol2, f0, npq, rz); break;
+    default: launch_update<64, T>(h, k, tol2, f0, npq, rz); break;
   }
 }
 
-void launch_sell_dot(Handle& h) {
+unsigned launch_sell_dot(Handle& h) {
   const Csr& A = h.A;
   if (A.srow.size() || A.sell_g != 1)
     fail(FEM_ERR_STATE, "the operator's sliced-ELL copy must keep the row order with one lane per row");
@@ -2036,64 +2113,64 @@ void launch_sell_dot(Handle& h) {
       blocks = nb;
     });
     HIP_LAUNCH_CHECK();
-    finish(h, (int)blocks, 1, F_ALPHA, 0);
-    return;
+    return blocks;
   }
   unsigned g = grid_for(A.nslices, kNT / 64);
   pcg_sell_dot_kernel<<<g, kNT, 0, h.stream>>>(A.n, A.nslices, sell_view(A), A.s64.get(), h.kp.get(), h.kq.get(),
                                                h.partials.get());
   HIP_LAUNCH_CHECK();
-  finish(h, (int)g, 1, F_ALPHA, 0);
+  return (unsigned)g;
 }
 
 template <int G>
-void launch_spmv_dot(Handle& h) {
+unsigned launch_spmv_dot(Handle& h) {
   const Csr& A = h.A;
   int64_t g = (A.n * G + kNT - 1) / kNT;
   if (g > 4096) g = 4096;
   pcg_spmv_dot_kernel<G><<<(unsigned)g, kNT, 0, h.stream>>>(A.n, A.rp.get(), A.ci.get(), A.v64.get(), h.kp.get(),
                                                             h.kq.get(), h.partials.get());
   HIP_LAUNCH_CHECK();
-  finish(h, (int)g, 1, F_ALPHA, 0);
+  return (unsigned)g;
 }
 
 template <int L>
-void launch_spmm_dot(Handle& h, int k) {
+unsigned launch_spmm_dot(Handle& h, int k) {
   const Csr& A = h.A;
   int64_t g = (A.n * L + kNT - 1) / kNT;
   if (g > 4096) g = 4096;
   pcg_spmm_dot_vec_kernel<L><<<(unsigned)g, kNT, 0, h.stream>>>(A.n, k, A.rp.get(), A.ci.get(), A.v64.get(), h.kp.get(),
                                                                 h.kq.get(), h.partials.get());
   HIP_LAUNCH_CHECK();
-  finish(h, (int)g, k, F_ALPHA, 0);
+  return (unsigned)g;
 }
 
-void spmv_dot(Handle& h, int k) {
+// q = A p; returns the count of p.q partials per column
+unsigned spmv_dot(Handle& h, int k) {
   const Csr& A = h.A;
   ProfScope ps(h, "pcg_spmv", matrix_bytes<double>(A, k) + 3.0 * 8 * A.n * k);
   if (k == 1 && A.nslices > 0 && A.s64.size() && A.sell_g == 1 && A.srow.size() == 0) {
-    launch_sell_dot(h);
+    return launch_sell_dot(h);
   } else if (k == 1) {
     switch (lanes_for(A)) {
-      case 4: launch_spmv_dot<4>(h); break;
-      case 8: launch_spmv_dot<8>(h); break;
-      case 16: launch_spmv_dot<16>(h); break;
-      case 32: launch_spmv_dot<32>(h); break;
-      default: launch_spmv_dot<64>(h); break;
+      case 4: return launch_spmv_dot<4>(h);
+      case 8: return launch_spmv_dot<8>(h);
+      case 16: return launch_spmv_dot<16>(h);
+      case 32: return launch_spmv_dot<32>(h);
+      default: return launch_spmv_dot<64>(h);
     }
   } else if (multi_staged<double>(A, k) && A.srow.size() == 0) {
     launch_lds_multi<double, kAssign, 1>(A, k, h.kp.get(), h.kq.get(), nullptr, (const double*)nullptr, nullptr,
                                          nullptr, 0.0, 0.0, nullptr, h.partials.get(), h.stream);
     HIP_LAUNCH_CHECK();
-    finish(h, (int)multi_blocks(A), k, F_ALPHA, 0);
+    return multi_blocks(A);
   } else {
     switch (pow2_at_least(k / 2)) {
-      case 1: launch_spmm_dot<1>(h, k); break;
-      case 2: launch_spmm_dot<2>(h, k); break;
-      case 4: launch_spmm_dot<4>(h, k); break;
-      case 8: launch_spmm_dot<8>(h, k); break;
-      case 16: launch_spmm_dot<16>(h, k); break;
-      default: launch_spmm_dot<32>(h, k); break;
+      case 1: return launch_spmm_dot<1>(h, k);
+      case 2: return launch_spmm_dot<2>(h, k);
+      case 4: return launch_spmm_dot<4>(h, k);
+      case 8: return launch_spmm_dot<8>(h, k);
+      case 16: return launch_spmm_dot<16>(h, k);
+      default: return launch_spmm_dot<32>(h, k);
     }
   }
 }
@@ -2207,22 +2284,22 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
     First0<float> f32 = first0_for<float>(h, k);
     const First0<double> f64 = first0_for<double>(h, k);
     if (!f32.on && h.H.precision >= 1 && !fused_level0(h, k, true)) f32.b = h.H.levels[0]->b32.get();
-    auto update_all = [&]() {  // x, r, rr, act
-      if (f64.on) update<double>(h, k, tol2, f64);
-      else update<float>(h, k, tol2, f32);
+    auto operator_update = [&](int rz) {  // q = A p, alpha; x, r, rr, act
+      const unsigned npq = spmv_dot(h, k);
+      if (f64.on) update<double>(h, k, tol2, f64, npq, rz);
+      else update<float>(h, k, tol2, f32, npq, rz);
     };
     while (any) {
-      // z = M r and rz = r.z (fused into the last level-0 smoothing step when
-      // possible); z stays where the preconditioner left it
-      auto precondition_dot = [&](int mode, int slot, bool r32_ready) {
-        const PrecOut o = precondition_pcg(h, h.kr.get(), h.kz.get(), k, h.partials.get(),
+      // z = M r and partials of r.z (fused into the last level-0 smoothing step
+      // when possible); z stays where the preconditioner left it
+      auto precondition_dot = [&](bool r32_ready) {
+        PrecOut o = precondition_pcg(h, h.kr.get(), h.kz.get(), k, h.partials.get(),
                                            r32_ready && f32.b, r32_ready && (f32.on || f64.on));
-        if (o.nb) finish(h, (int)o.nb, k, mode, slot);
-        else if (o.z32) dot(h, k, h.kr.get(), o.z32, mode, slot);
-        else dot(h, k, h.kr.get(), o.z64, mode, slot);
+        if (!o.nb) o.nb = o.z32 ? dot_partials(h, k, h.kr.get(), o.z32) : dot_partials(h, k, h.kr.get(), o.z64);
         return o;
       };
-      const PrecOut o0 = precondition_dot(F_STORE, S_RZ, false);
+      const PrecOut o0 = precondition_dot(false);
+      finish(h, (int)o0.nb, k, F_STORE, S_RZ);
       if (o0.z32) convert_kernel<float, double><<<grid_for(m, 256), 256, 0, s>>>(m, o0.z32, h.kp.get());
       else copy_kernel<<<grid_for(m, 256), 256, 0, s>>>(m, o0.z64, h.kp.get());
       HIP_LAUNCH_CHECK();
@@ -2233,7 +2310,19 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
       const bool flexible = cycle_type(h) == kCycleF;
       auto iteration = [&]() {
         // z, beta, rz
-        const PrecOut o = flexible ? precondition_dot(F_STORE, S_RZN, true) : precondition_dot(F_BETA, 0, true);
+        const PrecOut o = precondition_dot(true);
+        if (!flexible && folds(h, k, o.nb)) {
+          const unsigned g = grid_for(n, kNT);
+          if (o.z32)
+            pcg_p_fold_kernel<float><<<g, kNT, 0, s>>>(n, o.z32, h.kp.get(), h.scal.get(), h.partials.get(), (int)o.nb);
+          else
+            pcg_p_fold_kernel<double><<<g, kNT, 0, s>>>(n, o.z64, h.kp.get(), h.scal.get(), h.partials.get(),
+                                                        (int)o.nb);
+          HIP_LAUNCH_CHECK();
+          operator_update(S_RZN);
+          return;
+        }
+        finish(h, (int)o.nb, k, flexible ? F_STORE : F_BETA, flexible ? S_RZN : 0);
         if (flexible) {
           if (o.z32) dot(h, k, h.kq.get(), o.z32, F_FLEX, 0);
           else dot(h, k, h.kq.get(), o.z64, F_FLEX, 0);
@@ -2243,8 +2332,7 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
         else
           pcg_p_kernel<double><<<grid_for(m, 256), 256, 0, s>>>(m, k, o.z64, h.kp.get(), h.scal.get());
         HIP_LAUNCH_CHECK();
-        spmv_dot(h, k);           // q = A p, alpha
-        update_all();
+        operator_update(S_RZ);
       };
       // Iteration n ends with the n-th |r|^2 finish of this solve; the host
       // reads its record while iteration n + 1 may already run: the next
@@ -2255,8 +2343,7 @@ int pcg_solve(Handle& h, int k, fem_solve_info* info) {
       const uint64_t seq0 = seq_issued;
       auto issue = [&](bool first) {
         if (first) {
-          spmv_dot(h, k);
-          update_all();
+          operator_update(S_RZ);
         } else {
           run_iteration(h, k, tol2, iteration);
         }
