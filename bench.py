@@ -127,7 +127,7 @@ def cheb_step_bytes(n, nnz):
     return int(nnz * 8 + 4 * (n + 1) + n * 8 + n * 8 + n * 8)
 
 
-DOMINANT_KERNEL = "sell_lds_kernel<float, 4>"  # level-0 Chebyshev step (FP32 LDS-staged sliced ELL, fused epilogue)
+DOMINANT_KERNEL = "sell_lds_kernel<float, 4, 16>"  # level-0 Chebyshev step (FP32 LDS-staged sliced ELL, fused epilogue)
 TRAFFIC_FILE = ROOT / "profiles" / "traffic_level0_chebyshev_step.json"
 
 
