@@ -497,6 +497,13 @@ __global__ void __launch_bounds__(64 * kRowWaves) sym_wave_kernel(int64_t nrows,
   }
 }
 
+// orders this wavefront's LDS accesses before it ahead of those after it, for
+// values that pass between its lanes
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // cap: LDS slots per wavefront (the longest row); longer rows search their
 // columns and accumulate in memory (blocks of one wavefront only)
 __global__ void __launch_bounds__(64 * kRowWaves) num_wave_kernel(
@@ -530,10 +537,13 @@ __global__ void __launch_bounds__(64 * kRowWaves) num_wave_kernel(
       int at[kWaveUnroll];
 #pragma unroll
       for (int u = 0; u < kWaveUnroll; ++u) at[u] = B.c[u] >= 0 ? bsearch_col(s_cols, len, B.c[u]) : 0;
-      // one L entry after the other: one wavefront's LDS accesses execute in
-      // program order, so a column's next term follows its last
+      // one L entry after the other: a column's next term, on another lane,
+      // follows its last through the fence (a wavefront's LDS accesses execute
+      // in program order, so it costs no instruction; it keeps the compiler
+      // from reordering them)
 #pragma unroll
       for (int u = 0; u < kWaveUnroll; ++u) {
+        wave_lds_fence();
         if (B.c[u] >= 0) s_acc[at[u]] += a[u] * v[u];
         for (int q = B.s[u] + 64 + lane; q < B.e[u]; q += 64) s_acc[bsearch_col(s_cols, len, r_ci[q])] += a[u] * r_v[q];
       }
