@@ -21,6 +21,7 @@ struct FemError : public std::runtime_error {
 
 inline void hip_check(hipError_t e, const char* what, const char* file, int line) {
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // reported here, not by the next launch's check
     char buf[512];
     std::snprintf(buf, sizeof(buf), "HIP error %d (%s) in %s at %s:%d", (int)e,
                   hipGetErrorString(e), what, file, line);

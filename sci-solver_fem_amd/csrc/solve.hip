@@ -1954,6 +1954,7 @@ void ensure_krylov(Handle& h, int k) {
   }
   if (h.kcap < k) {
     ++h.gen;
+    h.kcap = 0;  // until all are there: an allocation that fails leaves some empty
     h.kx.resize(n * k); h.kr.resize(n * k); h.kp.resize(n * k); h.kq.resize(n * k);
     h.kz.resize(n * k); h.kb.resize(n * k);
     h.ubuf.resize(n * k); h.ubuf2.resize(n * k);
@@ -1971,6 +1972,7 @@ void ensure_krylov(Handle& h, int k) {
     Level& L = *Lp;
     if (L.wk >= k) continue;
     ++h.gen;
+    L.wk = 0;
     const int64_t nl = (&L == h.H.levels[0].get()) ? h.A.n : L.A.n;
     if (h.H.precision == 0) {
       L.x64.resize(nl * k); L.t64.resize(nl * k); L.b64.resize(nl * k); L.r64.resize(nl * k); L.d64.resize(nl * k);
