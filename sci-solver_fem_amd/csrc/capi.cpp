@@ -171,14 +171,14 @@ bool params_shape_changed(const fem_params& a, const fem_params& b) {
 void ensure_setup(Handle& h) {
   if (h.A.n == 0) fail(FEM_ERR_EMPTY, "Error no matrix specified");
   if (!h.H.built) {
-    DevPoolScope pool(h.stream);  // the setup's temporaries reuse each other's blocks
+    DevPoolScope pool(h.stream, !h.captured);  // the setup's temporaries reuse each other's blocks
     build_hierarchy(h);
   }
 }
 
 // work vectors for k (padded) columns, allocated like the setup's buffers
 void ensure_work(Handle& h, int k) {
-  DevPoolScope pool(h.stream);
+  DevPoolScope pool(h.stream, !h.captured);
   ensure_krylov(h, k);
 }
 
@@ -299,8 +299,9 @@ void fem_release_cached_memory(void) { pool_flush_reserve(); }
 void fem_destroy(fem_handle* hh) {
   Handle* h = H(hh);
   if (!h) return;
-  // with the handle's stream drained its buffers are idle and can be reused
-  const bool idle = h->stream && hipStreamSynchronize(h->stream) == hipSuccess;
+  // with the handle's stream drained its buffers are idle and can be reused,
+  // unless a caller's graph runs on them
+  const bool idle = h->stream && hipStreamSynchronize(h->stream) == hipSuccess && !h->captured;
   DevRetireScope retire(idle ? h->device : -1);
   if (h->h_scal) (void)hipHostFree(h->h_scal);
   if (h->h_act) (void)hipHostFree(h->h_act);

@@ -56,7 +56,10 @@ void* dev_malloc(size_t bytes);   // hipMalloc; on failure the reserve is freed 
 
 class DevPoolScope {
  public:
-  explicit DevPoolScope(hipStream_t stream);  // the stream of all the scope's work
+  // stream: of all the scope's work.  adopt false: blocks of earlier scopes
+  // that are released in this one may be in use on other streams, so they go
+  // through hipFree, which waits for the device.
+  explicit DevPoolScope(hipStream_t stream, bool adopt = true);
   ~DevPoolScope();
   DevPoolScope(const DevPoolScope&) = delete;
   DevPoolScope& operator=(const DevPoolScope&) = delete;

@@ -18,6 +18,7 @@ struct Pool {
   std::unordered_map<void*, size_t> owned;  // blocks this pool may hand on -> size class
   std::multimap<size_t, void*> free_;       // released blocks by size class
   int device = 0;
+  bool adopt = true;                        // takes blocks of earlier scopes
 };
 
 thread_local Pool* g_pool = nullptr;
@@ -136,7 +137,7 @@ bool pool_release(void* p) {
   auto bt = blocks().find(p);
   if (bt == blocks().end()) return false;
   const Block b = bt->second;
-  if (pl && b.device == pl->device) {
+  if (pl && pl->adopt && b.device == pl->device) {
     // a block of an earlier scope (the hierarchy that a setup replaces): its
     // uses are on this scope's stream, before whatever the block serves next
     pl->owned.emplace(p, b.cls);
@@ -151,8 +152,9 @@ bool pool_release(void* p) {
   return false;
 }
 
-DevPoolScope::DevPoolScope(hipStream_t stream) : prev_(g_pool), stream_(stream) {
+DevPoolScope::DevPoolScope(hipStream_t stream, bool adopt) : prev_(g_pool), stream_(stream) {
   Pool* pl = new Pool();
+  pl->adopt = adopt;
   (void)hipGetDevice(&pl->device);
   g_pool = pl;
 }

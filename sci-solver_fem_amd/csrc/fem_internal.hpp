@@ -190,6 +190,10 @@ struct Handle {
   int graph_k = 0;
   double graph_tol2 = 0.0;
 
+  // a caller's graph has captured work on the handle's buffers: its launches
+  // may run on any stream (the buffers are then given back through hipFree)
+  bool captured = false;
+
   bool profiling = false;
   std::map<std::string, KernelStat> stats;
   std::vector<PendingTiming> pending;   // recorded, not yet read back

@@ -2466,6 +2466,9 @@ void apply_preconditioner_noalloc(Handle& h, const double* r_user, double* z_use
   for (auto& Lp : h.H.levels) ready = ready && Lp->wk >= 1;
   if (!ready) fail(FEM_ERR_STATE, "fem_apply_preconditioner_noalloc: work vectors missing; call fem_setup first");
   if (h.profiling) fail(FEM_ERR_STATE, "fem_apply_preconditioner_noalloc: profiling is enabled");
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  HIP_CHECK(hipStreamIsCapturing(h.stream, &cap));
+  if (cap != hipStreamCaptureStatusNone) h.captured = true;
   double* base = scratch_address(h.device);
   double* r = base;
   double* z = base + kNoAllocRows;

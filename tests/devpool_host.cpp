@@ -1,0 +1,106 @@
+// The device-memory pool (csrc/devpool.cpp) on the CPU: the HIP calls it makes
+// are stand-ins over a simulated device of limited size, whose addresses are
+// never touched.  Runs the scenario named on the command line; exits with 0,
+// or prints the check that failed.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.hpp"
+
+namespace {
+std::mutex g_mu;
+std::map<char*, size_t> g_live;
+size_t g_used = 0, g_limit = (size_t)64 << 30;
+int g_mallocs = 0, g_frees = 0;
+constexpr size_t kGiB = (size_t)1 << 30;
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t bytes) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (g_used + bytes > g_limit) return hipErrorOutOfMemory;
+  char* at = reinterpret_cast<char*>((uintptr_t)1 << 40);  // the first gap, so that addresses come again
+  for (auto& kv : g_live) {
+    if (at + bytes <= kv.first) break;
+    at = kv.first + kv.second;
+  }
+  g_live[at] = bytes;
+  g_used += bytes;
+  ++g_mallocs;
+  *p = at;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  auto it = g_live.find(static_cast<char*>(p));
+  if (it == g_live.end()) {
+    std::printf("free of an address that is not allocated\n");
+    std::_Exit(1);
+  }
+  g_used -= it->second;
+  g_live.erase(it);
+  ++g_frees;
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "simulated"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t*, unsigned) { return hipErrorNotSupported; }
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipErrorNotSupported; }
+}
+
+#define CHECK(c)                                     \
+  do {                                               \
+    if (!(c)) {                                      \
+      std::printf("line %d: %s\n", __LINE__, #c);    \
+      std::exit(1);                                  \
+    }                                                \
+  } while (0)
+
+using fem::DevBuf;
+using fem::DevPoolScope;
+
+namespace {
+
+// a block that a scope's owner keeps (a handle's buffer)
+DevBuf<char> kept_block(size_t bytes) {
+  DevPoolScope s(nullptr);
+  return DevBuf<char>(bytes);
+}
+
+// work captured by a caller may run on any stream: what its handle releases
+// goes through hipFree, which waits for the device, and is not handed on
+void foreign_work() {
+  DevBuf<char> old = kept_block(kGiB);
+  {
+    DevPoolScope s(nullptr, /*adopt=*/false);
+    old.release();
+    CHECK(g_frees == 1);
+    DevBuf<char> next(kGiB);
+    CHECK(g_mallocs == 2);
+  }
+  old = kept_block(2 * kGiB);
+  {
+    DevPoolScope s(nullptr);
+    old.release();
+    const int m = g_mallocs;
+    DevBuf<char> next(2 * kGiB);
+    CHECK(g_mallocs == m);  // reused in stream order
+  }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const char* what = argc > 1 ? argv[1] : "";
+  if (!std::strcmp(what, "foreign_work")) foreign_work();
+  else { std::printf("unknown scenario\n"); return 2; }
+  return 0;
+}
