@@ -45,14 +45,15 @@ inline void hip_check(hipError_t e, const char* what, const char* file, int line
 // draw from (hipFree of each cost 0.1-0.65 ms, and large frees slow the
 // allocations after them: a setup replacing a hierarchy of 1 M rows spent 10
 // of 30 ms in 117 hipFree and 3 in hipMalloc); the reserve is freed by
-// pool_flush_reserve (fem_release_cached_memory) and whenever an allocation
-// fails.  Blocks still held when the scope ends (buffers the phase keeps) go
+// pool_flush_reserve (fem_release_cached_memory), and it and the scope's free
+// blocks whenever an allocation fails.  Blocks still held when the scope ends (buffers the phase keeps) go
 // back to the reserve when their handle is destroyed (DevRetireScope), and by
 // hipFree when their owner releases them at any other time.
 void* pool_alloc(size_t bytes);   // null when no scope is active on this thread
 bool pool_release(void* p);       // false when p is not a free-able pool block
 void pool_flush_reserve();
-void* dev_malloc(size_t bytes);   // hipMalloc; on failure the reserve is freed and it tries again
+void* dev_malloc(size_t bytes);   // hipMalloc; on failure what this thread's scopes and the reserve hold
+                                  // free is given back and it tries again
 
 class DevPoolScope {
  public:
@@ -63,10 +64,6 @@ class DevPoolScope {
   ~DevPoolScope();
   DevPoolScope(const DevPoolScope&) = delete;
   DevPoolScope& operator=(const DevPoolScope&) = delete;
-
- private:
-  void* prev_;
-  hipStream_t stream_;
 };
 
 // While alive on a thread, pool blocks of `device` released there go to the

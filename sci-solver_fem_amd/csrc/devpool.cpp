@@ -6,6 +6,7 @@
 #include <mutex>
 #include <thread>
 #include <unordered_map>
+#include <unordered_set>
 
 #include "../../include/fem_mi355x.h"
 #include "common.hpp"
@@ -15,10 +16,12 @@ namespace fem {
 namespace {
 
 struct Pool {
-  std::unordered_map<void*, size_t> owned;  // blocks this pool may hand on -> size class
-  std::multimap<size_t, void*> free_;       // released blocks by size class
+  std::unordered_set<void*> own;       // blocks handed out by this pool
+  std::multimap<size_t, void*> free_;  // released blocks by size class
   int device = 0;
-  bool adopt = true;                        // takes blocks of earlier scopes
+  bool adopt = true;                   // takes blocks of earlier scopes
+  hipStream_t stream = nullptr;        // of all the scope's work
+  Pool* prev = nullptr;                // the enclosing scope
 };
 
 thread_local Pool* g_pool = nullptr;
@@ -82,10 +85,28 @@ void pool_flush_reserve() {
   }
 }
 
+namespace {
+// frees the released blocks that this thread's scopes hold (a setup that
+// replaces a hierarchy of other sizes holds all of the old one)
+void free_released() {
+  for (Pool* pl = g_pool; pl; pl = pl->prev) {
+    if (pl->free_.empty() || hipStreamSynchronize(pl->stream) != hipSuccess) continue;
+    std::lock_guard<std::mutex> lk(g_res_mu);
+    for (auto& kv : pl->free_) {
+      for (Pool* q = g_pool; q; q = q->prev) q->own.erase(kv.second);
+      blocks().erase(kv.second);
+      (void)hipFree(kv.second);
+    }
+    pl->free_.clear();
+  }
+}
+}  // namespace
+
 void* dev_malloc(size_t bytes) {
   void* p = nullptr;
   if (hipMalloc(&p, bytes) != hipSuccess) {
     (void)hipGetLastError();
+    free_released();
     pool_flush_reserve();
     HIP_CHECK(hipMalloc(&p, bytes));
   }
@@ -120,27 +141,19 @@ void* pool_alloc(size_t bytes) {
     std::lock_guard<std::mutex> lk(g_res_mu);
     blocks()[p] = Block{c, pl->device};
   }
-  pl->owned.emplace(p, c);
+  pl->own.insert(p);
   return p;
 }
 
 bool pool_release(void* p) {
   Pool* pl = g_pool;
-  if (pl) {
-    auto it = pl->owned.find(p);
-    if (it != pl->owned.end()) {
-      pl->free_.emplace(it->second, p);
-      return true;
-    }
-  }
   std::lock_guard<std::mutex> lk(g_res_mu);
   auto bt = blocks().find(p);
   if (bt == blocks().end()) return false;
   const Block b = bt->second;
-  if (pl && pl->adopt && b.device == pl->device) {
-    // a block of an earlier scope (the hierarchy that a setup replaces): its
-    // uses are on this scope's stream, before whatever the block serves next
-    pl->owned.emplace(p, b.cls);
+  if (pl && b.device == pl->device && (pl->adopt || pl->own.count(p))) {
+    // also a block of an earlier scope (the hierarchy that a setup replaces):
+    // its uses are on this scope's stream, before whatever it serves next
     pl->free_.emplace(b.cls, p);
     return true;
   }
@@ -152,10 +165,12 @@ bool pool_release(void* p) {
   return false;
 }
 
-DevPoolScope::DevPoolScope(hipStream_t stream, bool adopt) : prev_(g_pool), stream_(stream) {
+DevPoolScope::DevPoolScope(hipStream_t stream, bool adopt) {
   Pool* pl = new Pool();
-  pl->adopt = adopt;
   (void)hipGetDevice(&pl->device);
+  pl->adopt = adopt;
+  pl->stream = stream;
+  pl->prev = g_pool;
   g_pool = pl;
 }
 
@@ -165,7 +180,7 @@ DevPoolScope::~DevPoolScope() {
     // queued work may still use the blocks: they are handed on once the
     // scope's stream has drained (a device synchronization would also end
     // another thread's stream capture)
-    const bool idle = hipStreamSynchronize(stream_) == hipSuccess;
+    const bool idle = hipStreamSynchronize(pl->stream) == hipSuccess;
     std::lock_guard<std::mutex> lk(g_res_mu);
     for (auto& kv : pl->free_) {
       if (idle) {
@@ -176,8 +191,8 @@ DevPoolScope::~DevPoolScope() {
       }
     }
   }
+  g_pool = pl->prev;
   delete pl;
-  g_pool = static_cast<Pool*>(prev_);
 }
 
 DevRetireScope::DevRetireScope(int device) : prev_(g_retire) { g_retire = device; }

@@ -96,11 +96,42 @@ void foreign_work() {
   }
 }
 
+// a setup that replaces a hierarchy by one of other sizes, near the limit of
+// the device: the old blocks make room
+void failed_allocation() {
+  g_limit = 10 * kGiB;
+  DevBuf<char> old = kept_block(7 * kGiB);
+  DevBuf<char> other = kept_block(kGiB);
+  {
+    DevPoolScope outer(nullptr);
+    other.release();
+    DevPoolScope s(nullptr);
+    old.release();
+    DevBuf<char> next(9 * kGiB);  // fits without the two
+    CHECK(g_used == 9 * kGiB);
+    // the freed addresses are new blocks now, of their own sizes
+    next.release();
+    DevBuf<char> a(4 * kGiB), b(4 * kGiB);
+    CHECK(a.get() != b.get() && g_live.at(a.get()) == 4 * kGiB && g_live.at(b.get()) == 4 * kGiB);
+    a.release();
+    DevBuf<char> c(4 * kGiB);
+    CHECK(g_live.at(c.get()) == 4 * kGiB);
+  }
+  bool failed = false;
+  try {
+    DevBuf<char> more(11 * kGiB);
+  } catch (const fem::FemError& e) {
+    failed = e.status == 3;
+  }
+  CHECK(failed);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "foreign_work")) foreign_work();
+  else if (!std::strcmp(what, "failed_allocation")) failed_allocation();
   else { std::printf("unknown scenario\n"); return 2; }
   return 0;
 }
