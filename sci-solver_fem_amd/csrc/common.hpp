@@ -42,7 +42,7 @@ inline void hip_check(hipError_t e, const char* what, const char* file, int line
 // scope and releases in this one (the hierarchy that a setup replaces) are
 // reused alike.  When the scope ends its free blocks go, once the
 // stream has drained, to a per-device reserve of at most 16 GiB that later scopes
-// draw from (hipFree of each cost 0.1-0.65 ms, and large frees slow the
+// draw from, the oldest blocks freed beyond that (hipFree of each cost 0.1-0.65 ms, and large frees slow the
 // allocations after them: a setup replacing a hierarchy of 1 M rows spent 10
 // of 30 ms in 117 hipFree and 3 in hipMalloc); the reserve is freed by
 // pool_flush_reserve (fem_release_cached_memory), and it and the scope's free

@@ -41,8 +41,28 @@ size_t size_class(size_t bytes) {
 // to one (process-lifetime objects: handles may be destroyed at exit)
 constexpr size_t kReserveCap = (size_t)16 << 30;  // a 161^3 handle and its temporaries: about 12 GiB
 struct Reserve {
-  std::multimap<size_t, void*> blocks;
+  struct Idle {
+    void* p;
+    uint64_t age;
+  };
+  typedef std::multimap<size_t, Idle> Blocks;
+  Blocks blocks;                               // by size class
+  std::map<uint64_t, Blocks::iterator> by_age; // oldest first
   size_t bytes = 0;
+  uint64_t next = 0;
+
+  void put(size_t cls, void* p) {
+    by_age.emplace(next, blocks.emplace(cls, Idle{p, next}));
+    ++next;
+    bytes += cls;
+  }
+  void* take(Blocks::iterator it) {
+    void* p = it->second.p;
+    by_age.erase(it->second.age);
+    bytes -= it->first;
+    blocks.erase(it);
+    return p;
+  }
 };
 struct Block {
   size_t cls;
@@ -58,31 +78,30 @@ std::unordered_map<void*, Block>& blocks() {
   return *b;
 }
 
-// an idle block into its device's reserve, or freed when that is full (the
-// caller holds g_res_mu)
+void free_block(void* p) {
+  blocks().erase(p);
+  (void)hipFree(p);
+}
+
+// an idle block into its device's reserve, whose oldest blocks make room: what
+// a process works on now has the sizes of the newest ones (the caller holds
+// g_res_mu)
 void retire_locked(void* p, size_t cls, int device) {
   Reserve& r = reserves()[device];
-  if (r.bytes + cls <= kReserveCap) {
-    r.blocks.emplace(cls, p);
-    r.bytes += cls;
-  } else {
-    blocks().erase(p);
-    (void)hipFree(p);
+  if (cls > kReserveCap) {
+    free_block(p);
+    return;
   }
+  while (r.bytes + cls > kReserveCap) free_block(r.take(r.by_age.begin()->second));
+  r.put(cls, p);
 }
 
 }  // namespace
 
 void pool_flush_reserve() {
   std::lock_guard<std::mutex> lk(g_res_mu);
-  for (auto& dr : reserves()) {
-    for (auto& kv : dr.second.blocks) {
-      blocks().erase(kv.second);
-      (void)hipFree(kv.second);
-    }
-    dr.second.blocks.clear();
-    dr.second.bytes = 0;
-  }
+  for (auto& dr : reserves())
+    while (!dr.second.blocks.empty()) free_block(dr.second.take(dr.second.blocks.begin()));
 }
 
 namespace {
@@ -94,8 +113,7 @@ void free_released() {
     std::lock_guard<std::mutex> lk(g_res_mu);
     for (auto& kv : pl->free_) {
       for (Pool* q = g_pool; q; q = q->prev) q->own.erase(kv.second);
-      blocks().erase(kv.second);
-      (void)hipFree(kv.second);
+      free_block(kv.second);
     }
     pl->free_.clear();
   }
@@ -129,11 +147,7 @@ void* pool_alloc(size_t bytes) {
     auto rt = reserves().find(pl->device);
     if (rt != reserves().end()) {
       auto jt = rt->second.blocks.find(c);
-      if (jt != rt->second.blocks.end()) {
-        p = jt->second;
-        rt->second.blocks.erase(jt);
-        rt->second.bytes -= c;
-      }
+      if (jt != rt->second.blocks.end()) p = rt->second.take(jt);
     }
   }
   if (!p) {
@@ -186,8 +200,7 @@ DevPoolScope::~DevPoolScope() {
       if (idle) {
         retire_locked(kv.second, kv.first, pl->device);
       } else {
-        blocks().erase(kv.second);
-        (void)hipFree(kv.second);
+        free_block(kv.second);
       }
     }
   }

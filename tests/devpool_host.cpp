@@ -126,12 +126,34 @@ void failed_allocation() {
   CHECK(failed);
 }
 
+// the reserve keeps the newest blocks: a process that goes from one size to
+// another finds the blocks of its present size there
+void reserve_ages() {
+  for (int size = 1; size <= 4; ++size) {  // 10 GiB of each
+    for (int round = 0; round < 2; ++round) {
+      DevPoolScope s(nullptr);
+      const int m = g_mallocs;
+      std::vector<DevBuf<char>> v;
+      for (int i = 0; i < 10 * 4 / size; ++i) v.emplace_back((size_t)size * kGiB / 4);
+      CHECK(g_mallocs - m == (round == 0 ? 10 * 4 / size : 0));
+    }
+    CHECK(g_used <= 16 * kGiB);
+  }
+  // a block larger than the reserve leaves it as it is
+  const size_t held = g_used;
+  { DevPoolScope s(nullptr); DevBuf<char> big(17 * kGiB); }
+  CHECK(g_used == held);
+  fem::pool_flush_reserve();
+  CHECK(g_used == 0 && g_live.empty());
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const char* what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "foreign_work")) foreign_work();
   else if (!std::strcmp(what, "failed_allocation")) failed_allocation();
+  else if (!std::strcmp(what, "reserve_ages")) reserve_ages();
   else { std::printf("unknown scenario\n"); return 2; }
   return 0;
 }
