@@ -134,8 +134,8 @@ void fem_destroy(fem_handle* h);
  * of destroyed handles, are kept (at most 16 GiB per device) for later builds
  * and setups to reuse, instead of a hipFree each.  The reserve is also freed
  * whenever a library allocation fails.  For callers that need the memory for
- * their own allocations; must not overlap with a fem_create_*, fem_setup,
- * fem_solve or fem_destroy call. */
+ * their own allocations; any thread may call it at any time, also beside other
+ * threads' calls (the reserve holds only blocks that nothing uses). */
 void fem_release_cached_memory(void);
 
 /* Message of the last failure on h (or of the last failed create if h is NULL). */

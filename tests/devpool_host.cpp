@@ -2,6 +2,7 @@
 // are stand-ins over a simulated device of limited size, whose addresses are
 // never touched.  Runs the scenario named on the command line; exits with 0,
 // or prints the check that failed.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -147,6 +148,52 @@ void reserve_ages() {
   CHECK(g_used == 0 && g_live.empty());
 }
 
+// fem_release_cached_memory beside setups, solves and destroys of other
+// threads: no block is ever with two owners, and none is lost
+void flush_beside_work() {
+  std::mutex mu;
+  std::map<void*, int> owner;
+  std::atomic<bool> stop{false};
+  std::thread flusher([&] {
+    while (!stop) fem::pool_flush_reserve();
+  });
+  auto work = [&](int id) {
+    unsigned x = 12345u + (unsigned)id;
+    auto next = [&] { return (x = x * 1664525u + 1013904223u) >> 8; };
+    for (int round = 0; round < 300; ++round) {
+      std::vector<DevBuf<char>> kept;
+      {
+        DevPoolScope s(nullptr);
+        for (int i = 0; i < 20; ++i) {
+          DevBuf<char> b(((size_t)1 << (8 + next() % 4)) * 3);
+          {
+            std::lock_guard<std::mutex> lk(mu);
+            CHECK(owner.emplace(b.get(), id).second);
+          }
+          if (next() % 2) {
+            kept.push_back(std::move(b));
+          } else {
+            std::lock_guard<std::mutex> lk(mu);
+            owner.erase(b.get());
+            b.release();
+          }
+        }
+      }
+      fem::DevRetireScope r(0);
+      std::lock_guard<std::mutex> lk(mu);
+      for (auto& b : kept) owner.erase(b.get());
+      kept.clear();
+    }
+  };
+  std::vector<std::thread> th;
+  for (int id = 0; id < 4; ++id) th.emplace_back(work, id);
+  for (auto& t : th) t.join();
+  stop = true;
+  flusher.join();
+  fem::pool_flush_reserve();
+  CHECK(g_used == 0 && g_live.empty());
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -154,6 +201,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(what, "foreign_work")) foreign_work();
   else if (!std::strcmp(what, "failed_allocation")) failed_allocation();
   else if (!std::strcmp(what, "reserve_ages")) reserve_ages();
+  else if (!std::strcmp(what, "flush_beside_work")) flush_beside_work();
   else { std::printf("unknown scenario\n"); return 2; }
   return 0;
 }

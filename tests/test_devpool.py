@@ -22,7 +22,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["foreign_work", "failed_allocation", "reserve_ages"])
+@pytest.mark.parametrize("scenario", ["foreign_work", "failed_allocation", "reserve_ages", "flush_beside_work"])
 def test_devpool(program, scenario):
     r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
