@@ -261,13 +261,16 @@ class FEMSolver:
         return z
 
     def update_kappa(self, kappa):
+        """New coefficients (at least num_elements() of them; more are ignored)
+        and reassembly.  numpy, or a tensor: one on the solver's device stays there."""
+        if (kappa.size if isinstance(kappa, np.ndarray) else kappa.numel()) < self.num_elements():
+            raise ValueError(f"kappa must have {self.num_elements()} entries")
         if isinstance(kappa, np.ndarray):
             k = np.ascontiguousarray(kappa, dtype=np.float64)
         else:
             import torch
             kd = kappa.detach()
-            if (kd.is_cuda and kd.device.index == self._p.device == torch.cuda.current_device()
-                    and kd.numel() >= self.num_elements()):
+            if kd.is_cuda and kd.device.index == self._p.device == torch.cuda.current_device():
                 # stays on the device: through the host, 48 MB of coefficients took 13 ms
                 kd = kd.to(torch.float64).contiguous()
                 object.__setattr__(self, "_operator_gen", self._operator_gen + 1)
