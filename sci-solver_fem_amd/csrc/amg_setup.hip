@@ -384,25 +384,6 @@ __global__ void __launch_bounds__(kProNT) prolongator_kernel(int64_t n, const in
   }
 }
 
-// per-block partial sums of v_i^2; with dinv, v is first scaled in place
-// (v_i *= dinv_i) and the sum taken over the scaled values
-__global__ void sumsq_kernel(int64_t n, double* __restrict__ v, const double* __restrict__ dinv,
-                             double* __restrict__ part) {
-  __shared__ double s_buf[kNT];
-  double a = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kNT) {
-    double x = v[i];
-    if (dinv) {
-      x *= dinv[i];
-      v[i] = x;
-    }
-    a += x * x;
-  }
-  double t = block_sum(a, s_buf);
-  if (threadIdx.x == 0) part[blockIdx.x] = t;
-}
-
-
 __global__ void hash_vector_kernel(int64_t n, unsigned long long seed, double* __restrict__ v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -413,54 +394,165 @@ __global__ void hash_vector_kernel(int64_t n, unsigned long long seed, double* _
   v[i] = 0.5 + (double)(z >> 11) * (1.0 / 9007199254740992.0);
 }
 
-// v *= 1 / nrm with nrm = sqrt(sum of the nb = kNT partials) when nrm > 0 (a
-// zero or NaN norm leaves v as it is).  Every block adds the partials itself
-// (2 KB, one per thread, the same tree everywhere), block 0 keeps the norm:
-// a launch of one thread walking them took 5 to 7 us per step.
-__global__ void __launch_bounds__(kNT) scale_by_norm_kernel(int64_t n, const double* __restrict__ part,
-                                                          double* __restrict__ nrm, double* __restrict__ v) {
+// Lanczos iteration on D^-1 A, symmetric in the D inner product: u_j = b_j v_j
+// with v_j the j-th basis vector and b_j = ||u_j||_D, so that no pass only
+// scales a vector.  A step is the product w = A u_j and the two kernels below,
+// which pass partial sums on to each other (every block adds them up itself,
+// in the same order; a launch of its own for that took 5 to 7 us).
+constexpr int kLanczosBlocks = 1024;
+
+// per-block partials of u.w, or without w of ||u||_D^2
+__global__ void __launch_bounds__(kNT) lanczos_dot_kernel(int64_t n, const double* __restrict__ u,
+                                                        const double* __restrict__ w,
+                                                        const double* __restrict__ dinv, double* __restrict__ part) {
   __shared__ double s_buf[kNT];
-  __shared__ double s_nrm;
-  const double t = block_sum(part[threadIdx.x], s_buf);
-  if (threadIdx.x == 0) {
-    s_nrm = sqrt(t);
-    if (blockIdx.x == 0) nrm[0] = s_nrm;
-  }
-  __syncthreads();
-  const double a = s_nrm;
-  if (!(a > 0)) return;
-  for (int64_t i = (int64_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kNT) v[i] *= 1.0 / a;
+  double a = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kNT)
+    a += w ? u[i] * w[i] : u[i] * u[i] / dinv[i];
+  const double t = block_sum(a, s_buf);
+  if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// Spectral radius of D^-1 A by power iteration (upper part of the spectrum),
-// on the device with one read-back at the end.
-double estimate_rho(const Csr& A, const double* dinv, hipStream_t s, int iters = 15) {
+// u_{j+1} = (D^-1 w - a_j u_j) / b_j - (b_j / b_{j-1}) u_{j-1} in place of
+// u_{j-1}, with a_j = u_j.w / b_j^2; a_j and b_j go to ab[2j], ab[2j+1], the
+// partials of ||u_{j+1}||_D^2 to next.  A norm that is not positive ends the
+// iteration (u_{j+1} = 0).
+__global__ void __launch_bounds__(kNT) lanczos_step_kernel(int64_t n, int j, const double* __restrict__ dot,
+                                                         const double* __restrict__ nrm, double* __restrict__ ab,
+                                                         const double* __restrict__ u, const double* __restrict__ w,
+                                                         const double* __restrict__ dinv, double* __restrict__ up,
+                                                         double* __restrict__ next) {
+  __shared__ double s_buf[kNT];
+  __shared__ double s_a, s_b;
+  double d = 0.0, q = 0.0;
+  for (int t = threadIdx.x; t < (int)gridDim.x; t += kNT) {
+    d += dot[t];
+    q += nrm[t];
+  }
+  d = block_sum(d, s_buf);
+  q = block_sum(q, s_buf);
+  if (threadIdx.x == 0) {
+    s_b = sqrt(q);
+    s_a = q > 0.0 ? d / q : 0.0;
+    if (blockIdx.x == 0) {
+      ab[2 * j] = s_a;
+      ab[2 * j + 1] = s_b;
+    }
+  }
+  __syncthreads();
+  const double a = s_a, b = s_b;
+  const bool live = b > 0.0;
+  const double ib = live ? 1.0 / b : 0.0;
+  const double c = live && j > 0 ? b / ab[2 * j - 1] : 0.0;
+  double part = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * kNT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kNT) {
+    const double di = dinv[i];
+    double x = (di * w[i] - a * u[i]) * ib;
+    if (j > 0) x -= c * up[i];
+    if (!live) x = 0.0;
+    up[i] = x;
+    part += x * x / di;
+  }
+  part = block_sum(part, s_buf);
+  if (threadIdx.x == 0) next[blockIdx.x] = part;
+}
+
+// What the m x m tridiagonal matrix of a Lanczos iteration says about the top
+// of the spectrum: a[0..m), and beside it b[1..m], b[j] coupling j-1 and j
+// (b[m] to the vector that a further step would take).  rho: the growth of the
+// last of `iters` power steps from the same start.  top: the largest
+// eigenvalue theta plus the residual of its vector; an eigenvalue of the
+// operator lies within that residual of theta.
+Spectrum lanczos_top(const double* a, const double* b, int m, int iters) {
+  Spectrum s;
+  // power steps in the Lanczos basis
+  std::vector<double> z(m + 1, 0.0), y(m + 1, 0.0);
+  z[0] = 1.0;
+  s.rho = 0.0;
+  for (int it = 0; it < iters; ++it) {
+    double q = 0.0;
+    for (int i = 0; i <= m; ++i) {
+      y[i] = (i < m ? a[i] * z[i] : 0.0) + (i > 0 ? b[i] * z[i - 1] : 0.0) + (i < m ? b[i + 1] * z[i + 1] : 0.0);
+      q += y[i] * y[i];
+    }
+    s.rho = std::sqrt(q);
+    if (!(s.rho > 0.0)) break;
+    for (int i = 0; i <= m; ++i) z[i] = y[i] / s.rho;
+  }
+  // largest eigenvalue by bisection on the signs of the LDL^T pivots of T - x
+  double lo = a[0], hi = 0.0;
+  for (int i = 0; i < m; ++i) {
+    lo = std::max(lo, a[i]);
+    hi = std::max(hi, a[i] + (i > 0 ? b[i] : 0.0) + (i + 1 < m ? b[i + 1] : 0.0));
+  }
+  for (int it = 0; it < 100 && lo < hi; ++it) {
+    const double x = 0.5 * (lo + hi);
+    bool above = false;  // an eigenvalue above x
+    double p = 1.0;
+    for (int i = 0; i < m && !above; ++i) {
+      p = a[i] - x - (i > 0 ? b[i] * b[i] / p : 0.0);
+      above = !(p < 0.0);
+    }
+    (above ? lo : hi) = x;
+  }
+  const double theta = 0.5 * (lo + hi);
+  // its vector, by the rows of T from the first
+  double y0 = 0.0, y1 = 1.0, norm = 1.0;
+  for (int i = 0; i + 1 < m; ++i) {
+    const double y2 = ((theta - a[i]) * y1 - (i > 0 ? b[i] * y0 : 0.0)) / b[i + 1];
+    y0 = y1;
+    y1 = y2;
+    norm += y2 * y2;
+  }
+  s.top = theta + b[m] * std::fabs(y1) / std::sqrt(norm);
+  return s;
+}
+
+// The top of the spectrum of D^-1 A from 14 Lanczos steps, on the device with
+// one read-back at the end.  Where a few elements dominate (lognormal
+// coefficients) the largest eigenvalue is up to 1.29 times what a power
+// iteration of as many steps shows, and a Chebyshev interval that leaves it out
+// by more than 3 % makes the V-cycle indefinite: PCG then takes more iterations,
+// in a count that depends on rounding, or does not converge (with the interval
+// from 1.1 times the power iteration, and from this one: 61 x 58 x 73, sigma 1,
+// FP64 36 and 24 iterations, mixed 55 and 24; 500 x 400, sigma 1, mixed, five
+// columns none in 1000 and 36).
+Spectrum estimate_spectrum(const Csr& A, const double* dinv, hipStream_t s, int iters = 14) {
   const int64_t n = A.n;
-  const int nb = kNT;
-  DevBuf<double> v(n), w(n), part(nb), nrm(iters + 1);
-  hash_vector_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, 12345ull, v.get());
+  const int nb = (int)std::min<unsigned>(grid_for(n, kNT), (unsigned)kLanczosBlocks);
+  // a_j, b_j; partials of u.w; two of norms
+  DevBuf<double> u(n), up(n), w(n), buf(2 * iters + 3 * nb);
+  double* ab = buf.get();
+  double* dot = ab + 2 * iters;
+  double* nrm = dot + nb;
+  double* next = nrm + nb;
+  hash_vector_kernel<<<grid_for(n, 256), 256, 0, s>>>(n, 12345ull, u.get());
   HIP_LAUNCH_CHECK();
-  // x (scaled by `scale` first) over its norm, which goes to out
-  auto normalise = [&](double* x, const double* scale, double* out) {
-    sumsq_kernel<<<nb, kNT, 0, s>>>(n, x, scale, part.get());
+  lanczos_dot_kernel<<<nb, kNT, 0, s>>>(n, u.get(), nullptr, dinv, nrm);
+  HIP_LAUNCH_CHECK();
+  for (int j = 0; j < iters; ++j) {
+    spmv64(A, u.get(), w.get(), s);
+    lanczos_dot_kernel<<<nb, kNT, 0, s>>>(n, u.get(), w.get(), dinv, dot);
     HIP_LAUNCH_CHECK();
-    scale_by_norm_kernel<<<std::min<unsigned>(grid_for(n, kNT), 2048u), kNT, 0, s>>>(n, part.get(), out, x);
+    lanczos_step_kernel<<<nb, kNT, 0, s>>>(n, j, dot, nrm, ab, u.get(), w.get(), dinv, up.get(), next);
     HIP_LAUNCH_CHECK();
-  };
-  normalise(v.get(), nullptr, nrm.get());
-  for (int it = 0; it < iters; ++it) {
-    spmv64(A, v.get(), w.get(), s);
-    normalise(w.get(), dinv, nrm.get() + 1 + it);  // w = D^-1 A v over its norm
-    std::swap(v, w);
+    std::swap(u, up);
+    std::swap(nrm, next);
   }
-  std::vector<double> h = nrm.to_host(s);
-  // the last norm, or the first that was not positive (the iteration stops there)
-  double rho = 1.0;
-  for (int it = 0; it < iters; ++it) {
-    rho = h[1 + it];
-    if (!(rho > 0)) break;
+  const std::vector<double> h = buf.to_host(s);
+  std::vector<double> a(iters), b(iters + 1);
+  for (int j = 0; j < iters; ++j) {
+    a[j] = h[2 * j];
+    b[j] = h[2 * j + 1];
   }
-  return rho;
+  double q = 0.0;
+  for (int t = 0; t < nb; ++t) q += h[(nrm - ab) + t];
+  b[iters] = std::sqrt(q);
+  // an invariant subspace ends the iteration; b[0] is the start's norm
+  int m = 1;
+  while (m < iters && b[m] > 1e-12 * std::fabs(a[0])) ++m;
+  if (m < iters && !std::isnan(b[m])) b[m] = 0.0;
+  return lanczos_top(a.data(), b.data(), m, iters);
 }
 
 __global__ void lower_bound_u32_kernel(int64_t m, const uint32_t* __restrict__ keys, int64_t nk,
@@ -1114,7 +1206,7 @@ void build_hierarchy(Handle& h) {
       break;
     }
     L.nc = nagg;
-    L.rho = estimate_rho(A, L.dinv64.get(), s);
+    L.spec = estimate_spectrum(A, L.dinv64.get(), s);
     // prolongator pattern: columns agg(k) for k in row i of A
     if (!agg_pattern(A, L.agg.get(), nagg, L.P, s))
       spgemm_symbolic(A, nullptr, nullptr, 0, L.agg.get(), nagg, false, L.P, s);

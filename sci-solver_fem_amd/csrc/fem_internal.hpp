@@ -79,6 +79,12 @@ struct Csr {
   LdsList lds, ldm;
 };
 
+// The top of the spectrum of D^-1 A: rho, where a power iteration gets to; top,
+// at or above the largest eigenvalue as far as the setup's Lanczos steps show it
+struct Spectrum {
+  double rho = 2.0, top = 2.0;
+};
+
 struct Level {
   Csr A;
   DevBuf<double> dinv64;
@@ -87,7 +93,7 @@ struct Level {
   Csr R;                  // nc x n restriction = P^T
   DevBuf<int32_t> agg;    // n, aggregate of each row
   int64_t nc = 0;
-  double rho = 2.0;       // spectral radius estimate of D^-1 A
+  Spectrum spec;          // of D^-1 A
   // V-cycle work vectors (one RHS column block of width `wk`)
   int wk = 0;
   DevBuf<double> x64, t64, b64, r64, d64;
