@@ -272,7 +272,7 @@ class FEMSolver:
             kd = kappa.detach()
             if kd.is_cuda and kd.device.index == self._p.device == torch.cuda.current_device():
                 # stays on the device: through the host, 48 MB of coefficients took 13 ms
-                kd = kd.to(torch.float64).contiguous()
+                kd = kd.to(torch.float64).resolve_neg().contiguous()
                 object.__setattr__(self, "_operator_gen", self._operator_gen + 1)
                 self._bind_torch_stream()
                 _check(self._h, lib().fem_update_kappa_device(self._h, _ptr(kd)))

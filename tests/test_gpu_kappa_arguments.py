@@ -29,3 +29,19 @@ def test_short_kappa_is_refused(gpu, fem, form):
     s.update_kappa(np.concatenate([kappa, kappa[:3]]))  # more entries than elements: the first ones count
     assert np.array_equal(s.get_matrix_csr()[2], before)
     s.close()
+
+
+@pytest.mark.parametrize("form", ["imaginary", "contiguous"])
+def test_negated_view(gpu, fem, form):
+    """Tensors that store the negative of their values (the imaginary part of
+    a conjugate)."""
+    import torch
+    s, kappa = _solver(fem)
+    want = s.get_matrix_csr()[2]
+    t = torch.from_numpy(-kappa).cuda()
+    t = torch.complex(torch.zeros_like(t), t).conj().imag if form == "imaginary" else torch._neg_view(t)
+    assert t.is_neg() and t.is_contiguous() == (form == "contiguous")
+    s.update_kappa(np.ones_like(kappa))
+    s.update_kappa(t)
+    assert np.array_equal(s.get_matrix_csr()[2], want)
+    s.close()
