@@ -761,7 +761,9 @@ __global__ void __launch_bounds__(kNT) sell_multi_kernel(int64_t n, int k, int64
 // only by other wavefronts: full occupancy (at most 64 registers) beats loads
 // issued ahead (161^3, 16 columns, FP32 step 479 us unstaged, 417 staged; 476
 // with the row's vectors and entries loaded before the staging at 5 wavefronts
-// a SIMD).  FP64 rows of 16 columns have eight lanes; there the lanes of a
+// a SIMD).  A lane takes 16 bytes of columns, so that few lanes load each entry:
+// 161^3, 4 columns, FP32 step 161 us by one lane a row, 309 by four lanes of one
+// column each, 181 unstaged; FP64 301, 380 and 333.  FP64 rows of 16 columns have eight lanes; there the lanes of a
 // quad load one entry each of four and share them by DPP (operator + p.q 738
 // us unstaged, 747 staged with all lanes loading every code and value, the
 // address unit 70 % busy, 721 shared).  61 x 58 x 73, 5 columns in 8, FP64
@@ -800,7 +802,7 @@ __device__ __forceinline__ void quad_entries(int c, T v, int m, const Vec* xl, i
 template <typename T, int LN, typename Vec>
 __device__ __forceinline__ Vec multi_row_sum(const uint16_t* cp, const T* vp, int w, const Vec* xl) {
   Vec acc = (Vec)(T(0));
-  if constexpr (sizeof(T) == 8) {
+  if constexpr (sizeof(T) == 8 && LN >= 4) {
     const int q4 = threadIdx.x & 3;  // entry 4 g + q4 of the row is this lane's of group g
     for (int g = 0; 4 * g < w; ++g) {
       int ec = 0;
@@ -837,7 +839,7 @@ __global__ void __launch_bounds__(64 * kMultiSlices * LN, 8) sell_lds_multi_kern
     T* __restrict__ y, const T* __restrict__ b, const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ xn,
     T c1, T c2, const double* __restrict__ r64, double* __restrict__ partials) {
   typedef typename VecOf<T, VW>::type vec;
-  static_assert(LN >= 4 && 64 % LN == 0, "whole quads per row, rows of one slice per wavefront");
+  static_assert(64 % LN == 0, "rows of one slice per wavefront");
   extern __shared__ unsigned char lds_raw[];
   vec* xs = reinterpret_cast<vec*>(lds_raw);
   __shared__ double s_dot[DOT ? kMultiSlices * LN * VW * LN : 1];

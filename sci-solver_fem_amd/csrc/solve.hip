@@ -199,18 +199,18 @@ constexpr int kMultiLds = 122880;  // bytes of x rows a block stages at most
 
 const LdsList& multi_list(const Csr& A) { return A.ldm.bs > 0 ? A.ldm : A.lds; }
 
-// columns per lane and lanes per row: 16 FP32 columns by four lanes, 16 FP64
-// columns by eight (16 bytes a lane); 4 or 8 columns by four lanes.  Operators
+// columns per lane (16 bytes) and lanes per row: 4, 8 and 16 columns by one,
+// two and four lanes in FP32, twice as many in FP64.  Operators
 // with a staged copy take it whatever their row length (161^3 level 1, ~46
 // entries: 43.9 us a step against 52.2 for the entry-split CSR kernel)
 template <typename T>
-int multi_cols(int k) { return std::min(pow2_at_least(k / 4), 16 / (int)sizeof(T)); }
+constexpr int kMultiCols = 16 / (int)sizeof(T);
 template <typename T>
-int multi_lanes(int k) { return sizeof(T) == 8 && k > 8 ? 8 : 4; }
+int multi_lanes(int k) { return std::min(pow2_at_least(k / kMultiCols<T>), sizeof(T) == 8 ? 8 : 4); }
 
 template <typename T>
 size_t multi_lds(const Csr& A, int k) {
-  return (size_t)multi_list(A).maxc * multi_cols<T>(k) * multi_lanes<T>(k) * sizeof(T);
+  return (size_t)multi_list(A).maxc * kMultiCols<T> * multi_lanes<T>(k) * sizeof(T);
 }
 
 template <typename T>
@@ -226,24 +226,18 @@ template <typename T, int MODE, int DOT>
 void launch_lds_multi(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T* d, T* xn, T c1, T c2,
                       const double* r64, double* partials, hipStream_t s) {
   const LdsList& M = multi_list(A);
-  auto go = [&](auto vw, auto ln) {
-    constexpr int VW = decltype(vw)::value, LN = decltype(ln)::value;
+  auto go = [&](auto ln) {
+    constexpr int VW = kMultiCols<T>, LN = decltype(ln)::value;
     sell_lds_multi_kernel<T, VW, LN, MODE, DOT><<<multi_blocks(A), 64 * M.bs * LN, multi_lds<T>(A, k), s>>>(
         A.n, k, A.nslices, sell_view(A), lds_view(M), svals_of<T>(A), x, y, b, dinv, d, xn, c1, c2, r64, partials);
   };
-  using One = std::integral_constant<int, 1>;
-  using Two = std::integral_constant<int, 2>;
-  using Four = std::integral_constant<int, 4>;
-  using Eight = std::integral_constant<int, 8>;
-  const int vw = multi_cols<T>(k);
-  if (vw == 1)
-    go(One{}, Four{});
-  else if constexpr (sizeof(T) == 8) {
-    if (multi_lanes<T>(k) == 4) go(Two{}, Four{});
-    else go(Two{}, Eight{});
-  } else {
-    if (vw == 2) go(Two{}, Four{});
-    else go(Four{}, Four{});
+  switch (multi_lanes<T>(k)) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    default:
+      if constexpr (sizeof(T) == 8) go(std::integral_constant<int, 8>{});
+      break;
   }
 }
 
@@ -1933,10 +1927,11 @@ void apply_level_int(Handle& h, int lvl, int which, const double* x, double* y) 
 }
 
 int padded_columns(const Handle&, int k) {
-  // fours: whole 16-byte FP32 groups in every kernel.  5 columns in 8 against a
-  // lane per column with 3 of 8 idle (61 x 58 x 73, FP64 solve 16.4 -> 9.7 ms):
-  // the entry-split and staged kernels need groups, and the kernels that took
-  // any count walked the coarse levels' long rows serially (43 us for 832 rows)
+  // fours: whole 16-byte FP32 groups in every kernel.  Kernels for any count had
+  // a lane per column and walked the coarse levels' long rows serially (43 us
+  // for 832 rows).  An iteration of theirs, and of this one: 161^3 mixed, 2
+  // columns 3.36 and 1.84 ms, 5 columns 5.14 and 2.9; 61 x 58 x 73 FP64, 2
+  // columns 401 and 256 us, 3 columns 504 and 256, 5 columns 631 and 337.
   if (k <= 1) return 1;
   return (k + 3) / 4 * 4;
 }
