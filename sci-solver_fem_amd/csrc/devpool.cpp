@@ -46,22 +46,24 @@ struct Reserve {
     uint64_t age;
   };
   typedef std::multimap<size_t, Idle> Blocks;
-  Blocks blocks;                               // by size class
-  std::map<uint64_t, Blocks::iterator> by_age; // oldest first
+  Blocks blocks;  // by size class
   size_t bytes = 0;
   uint64_t next = 0;
 
   void put(size_t cls, void* p) {
-    by_age.emplace(next, blocks.emplace(cls, Idle{p, next}));
-    ++next;
+    blocks.emplace(cls, Idle{p, next++});
     bytes += cls;
   }
   void* take(Blocks::iterator it) {
     void* p = it->second.p;
-    by_age.erase(it->second.age);
     bytes -= it->first;
     blocks.erase(it);
     return p;
+  }
+  Blocks::iterator oldest() {  // only a full reserve asks, before a hipFree
+    return std::min_element(blocks.begin(), blocks.end(), [](const Blocks::value_type& a, const Blocks::value_type& b) {
+      return a.second.age < b.second.age;
+    });
   }
 };
 struct Block {
@@ -92,7 +94,7 @@ void retire_locked(void* p, size_t cls, int device) {
     free_block(p);
     return;
   }
-  while (r.bytes + cls > kReserveCap) free_block(r.take(r.by_age.begin()->second));
+  while (r.bytes + cls > kReserveCap) free_block(r.take(r.oldest()));
   r.put(cls, p);
 }
 
