@@ -502,7 +502,7 @@ int fem_solve(fem_handle* hh, const double* b, double* x, int nrhs, int on_devic
       ensure_setup(h);
       setup_ms = h.H.setup_ms;
     }
-    const int kk = padded_columns(h, nrhs);
+    const int kk = padded_columns(nrhs, h.H.precision == 0);
     ensure_work(h, kk);
     to_internal(h, b, on_device, h.kb.get(), nrhs, kk);
     to_internal(h, x, on_device, h.kx.get(), nrhs, kk);
@@ -576,7 +576,7 @@ int fem_apply_operator(fem_handle* hh, const double* x, double* y, int nrhs, int
   return guarded(hh, [&]() {
     Handle& h = *H(hh);
     if (h.A.n == 0) fail(FEM_ERR_EMPTY, "Error no matrix specified");
-    const int kk = padded_columns(h, nrhs);
+    const int kk = padded_columns(nrhs, true);
     ensure_work(h, kk);
     to_internal(h, x, on_device, h.kp.get(), nrhs, kk);
     apply_operator_int(h, h.kp.get(), h.kq.get(), kk);

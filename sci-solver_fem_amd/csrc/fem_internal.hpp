@@ -276,8 +276,9 @@ void aggregate_graph(int64_t n, const int32_t* adj_ptr, const int32_t* adj, int 
 
 // ---- solve (solve.hip) ----
 // columns the kernels hold for k right-hand sides: k padded with zero columns
-// (a zero right-hand side starts, and stays, converged)
-int padded_columns(const Handle& h, int k);
+// (a zero right-hand side starts, and stays, converged); fp64: all of the work
+// is in FP64
+int padded_columns(int k, bool fp64);
 void ensure_krylov(Handle& h, int k);  // k padded
 int pcg_solve(Handle& h, int k, fem_solve_info* info);   // uses h.kb (rhs), h.kx (x0 / out), internal order
 void apply_vcycle_fp64(Handle& h, const double* r, double* z);  // level-0 preconditioner, 1 column

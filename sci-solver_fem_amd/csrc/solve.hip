@@ -216,7 +216,7 @@ size_t multi_lds(const Csr& A, int k) {
 template <typename T>
 bool multi_staged(const Csr& A, int k) {
   const LdsList& M = multi_list(A);
-  return k > 1 && k % 4 == 0 && A.nslices > 0 && A.sell_g == 1 && svals_of<T>(A) && M.bs > 0 &&
+  return k > 1 && k % kMultiCols<T> == 0 && A.nslices > 0 && A.sell_g == 1 && svals_of<T>(A) && M.bs > 0 &&
          M.bs <= kMultiSlices && multi_lds<T>(A, k) <= (size_t)kMultiLds;
 }
 
@@ -1926,14 +1926,16 @@ void apply_level_int(Handle& h, int lvl, int which, const double* x, double* y) 
   }
 }
 
-int padded_columns(const Handle&, int k) {
-  // fours: whole 16-byte FP32 groups in every kernel.  Kernels for any count had
-  // a lane per column and walked the coarse levels' long rows serially (43 us
-  // for 832 rows).  An iteration of theirs, and of this one: 161^3 mixed, 2
-  // columns 3.36 and 1.84 ms, 5 columns 5.14 and 2.9; 61 x 58 x 73 FP64, 2
-  // columns 401 and 256 us, 3 columns 504 and 256, 5 columns 631 and 337.
+int padded_columns(int k, bool fp64) {
+  // whole 16-byte groups: pairs in FP64, fours where FP32 vectors take part.
+  // Kernels for any count had a lane per column and walked the coarse levels'
+  // long rows serially (43 us for 832 rows).  An iteration of theirs, of fours
+  // in every precision, and of this rule: 161^3 FP64, 2 columns 4.55, 3.60 and
+  // 1.96 ms, 6 columns 5.71, 4.40 and 4.04; 1003 x 701 FP64, 6 columns 626, 713
+  // and 577 us; 161^3 mixed, 2 columns 3.36 and 1.84 ms, 5 columns 5.14 and 2.9.
   if (k <= 1) return 1;
-  return (k + 3) / 4 * 4;
+  const int g = fp64 ? 2 : 4;
+  return (k + g - 1) / g * g;
 }
 
 void ensure_krylov(Handle& h, int k) {
