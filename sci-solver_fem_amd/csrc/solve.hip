@@ -280,8 +280,7 @@ void spmv_op(const Csr& A, int k, const T* x, T* y, const T* b, const T* dinv, T
       case 2: launch_sell_multi<T, MODE, 2>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
       case 4: launch_sell_multi<T, MODE, 4>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
       case 8: launch_sell_multi<T, MODE, 8>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
-      case 16: launch_sell_multi<T, MODE, 16>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
-      default: launch_sell_multi<T, MODE, 32>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
+      default: launch_sell_multi<T, MODE, 16>(A, k, x, y, b, dinv, d, xn, c1, c2, s); break;
     }
   } else {
     // 16-byte column groups (all multi-column vectors here come from hipMalloc;

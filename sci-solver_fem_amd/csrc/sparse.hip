@@ -436,7 +436,7 @@ struct WaveBatch {
 };
 
 template <bool kFill>
-__global__ void __launch_bounds__(64 * kRowWaves) sym_wave_kernel(int64_t nrows, const int32_t* __restrict__ l_rp,
+__global__ void __launch_bounds__(64 * kRowWaves) sym_wave_kernel(const int32_t* __restrict__ l_rp,
                                                     const int32_t* __restrict__ l_ci,
                                                     const int32_t* __restrict__ r_rp,
                                                     const int32_t* __restrict__ r_ci,
@@ -507,7 +507,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // cap: LDS slots per wavefront (the longest row); longer rows search their
 // columns and accumulate in memory (blocks of one wavefront only)
 __global__ void __launch_bounds__(64 * kRowWaves) num_wave_kernel(
-    int64_t nrows, int cap, const int32_t* __restrict__ l_rp, const int32_t* __restrict__ l_ci,
+    int cap, const int32_t* __restrict__ l_rp, const int32_t* __restrict__ l_ci,
     const double* __restrict__ l_v, const int32_t* __restrict__ r_rp, const int32_t* __restrict__ r_ci,
     const double* __restrict__ r_v, const int32_t* __restrict__ c_rp, const int32_t* __restrict__ c_ci,
     double* __restrict__ c_v) {
@@ -1157,14 +1157,14 @@ void spgemm_symbolic(const Csr& L, const int32_t* r_rp, const int32_t* r_ci, int
   if (use_wave_rows(n, ncols)) {
     const size_t lds = sizeof(unsigned) * (size_t)((ncols + 31) / 32 > 0 ? (ncols + 31) / 32 : 1);
     DevBuf<int32_t> cnt(n);
-    sym_wave_kernel<false><<<(unsigned)n, 64 * row_waves(n), lds, s>>>(n, L.rp.get(), L.ci.get(), r_rp, r_ci, colmap,
+    sym_wave_kernel<false><<<(unsigned)n, 64 * row_waves(n), lds, s>>>(L.rp.get(), L.ci.get(), r_rp, r_ci, colmap,
                                                         drop_diag ? 1 : 0, ncols, cnt.get(), nullptr, nullptr);
     HIP_LAUNCH_CHECK();
     int64_t nnz = dev_exclusive_scan_i32(cnt.get(), C.rp.get(), n, s);
     if (nnz >= ((int64_t)1 << 31)) fail(FEM_ERR_CAPACITY, "sparse product has 2^31 or more nonzeros");
     C.nnz = nnz;
     C.ci.resize(nnz > 0 ? nnz : 1);
-    sym_wave_kernel<true><<<(unsigned)n, 64 * row_waves(n), lds, s>>>(n, L.rp.get(), L.ci.get(), r_rp, r_ci, colmap,
+    sym_wave_kernel<true><<<(unsigned)n, 64 * row_waves(n), lds, s>>>(L.rp.get(), L.ci.get(), r_rp, r_ci, colmap,
                                                        drop_diag ? 1 : 0, ncols, cnt.get(), C.rp.get(), C.ci.get());
     HIP_LAUNCH_CHECK();
     HIP_CHECK(hipStreamSynchronize(s));
@@ -1295,7 +1295,7 @@ void spgemm_numeric(const Csr& L, const Csr& Rm, Csr& C, hipStream_t s) {
     int waves = maxlen <= wcap ? row_waves(C.n) : 1;
     while (waves > 1 && wcap * (8 * waves + 4) > 61440) waves /= 2;
     num_wave_kernel<<<(unsigned)C.n, 64 * waves, (size_t)wcap * (8 * waves + 4), s>>>(
-        C.n, wcap, L.rp.get(), L.ci.get(), L.v64.get(), Rm.rp.get(), Rm.ci.get(), Rm.v64.get(), C.rp.get(),
+        wcap, L.rp.get(), L.ci.get(), L.v64.get(), Rm.rp.get(), Rm.ci.get(), Rm.v64.get(), C.rp.get(),
         C.ci.get(), C.v64.get());
     HIP_LAUNCH_CHECK();
     return;
