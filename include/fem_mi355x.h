@@ -254,10 +254,11 @@ int fem_get_level_prolongator(const fem_handle* h, int lvl, int64_t* nnz,
  * diagnostic hook beside the level exports above (the reference applies these
  * matrices inside AMG_Level::cycle, src/core/cuda/amg_level.cu:22-128). */
 int fem_apply_level(fem_handle* h, int lvl, int which, const double* x, double* y);
-/* Smoother data of level lvl (not the coarsest): rho, the power-iteration
- * estimate of rho(D^-1 A); the Chebyshev interval [lmin, lmax] =
- * [1.1 rho / 30, 1.1 rho] and the Jacobi weight omega = smootherWeight *
- * 4 / (3 rho) derived from it.  Any output may be NULL.  Diagnostic hook; the
+/* Smoother data of level lvl (not the coarsest): rho, the estimate of
+ * rho(D^-1 A) that a power iteration gives; the Chebyshev interval
+ * [lmin, lmax], lmax = max(1.1 rho, largest Ritz value + its residual) and
+ * lmin = lmax / 30; the Jacobi weight omega = smootherWeight * 4 / (3 rho).
+ * All from 14 Lanczos steps at setup.  Any output may be NULL.  Diagnostic hook; the
  * reference's smoother has a fixed weight (src/core/cuda/gauss_seidel.cu:1279-1376). */
 int fem_get_level_smoother(const fem_handle* h, int lvl, double* rho, double* lmin, double* lmax,
                            double* omega);

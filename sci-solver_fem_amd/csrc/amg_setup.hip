@@ -313,7 +313,7 @@ void randomized_mis(int64_t n, const int32_t* adj_ptr, const int32_t* adj, int d
   }
 }
 
-// ---- prolongator, diagonal, power iteration ---------------------------------------
+// ---- prolongator, diagonal, Lanczos iteration -------------------------------------
 
 __global__ void diag_kernel(int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
                             const double* __restrict__ v, double* __restrict__ dinv, int* __restrict__ bad) {
@@ -1105,7 +1105,7 @@ void build_hierarchy(Handle& h) {
   // level-0 graph: pattern of A without the diagonal
   Csr G;
   if (h.prm.strengthThreshold <= 0.0) offdiag_graph(h.A, G, s);
-  // the fine operator's sliced copy first (the power iteration below runs on
+  // the fine operator's sliced copy first (the Lanczos steps below run on
   // it), with its diagonal outside the slices: the diagonal term then needs
   // no column code and no gather (x_i is read by the row anyway; measured
   // 3-5 % per level-0 pass at 161^3)
